@@ -128,10 +128,6 @@ __device__ __forceinline__ void pp_strip_store(int i, const int32_t* region, con
     const int ml = wm * C::WTM + i * 32 + row;
     const int m = m0 + ml;
     const float rv = sc_row[ml];
-    if (ORDER < 0 && order == LSK_EPI_V25) {  // the outlier side term needs (m, n): operands from memory
-      if (m < M && n < N) epilogue_store4(ep, m, n, N, v, vec);
-      continue;
-    }
     if (m < M && n < N)
       epilogue_store4_pre(ep.out, ep.ldo, order, odt, has_bias, ep.shift, m, n, N, v, rv, wsv, bv,
                           pow2 ? __float_as_int(rv) : 0, ecv, vec);
@@ -229,11 +225,109 @@ __device__ __forceinline__ void pp_epilogue(const typename C::Acc& acc, const Ep
   }
 }
 
+// LDS of the V25 side term of a tile: kJC declared channels at a time, ho as [BM][kJC + 1] and wo
+// as [kJC][BN + 4] binary32 (the paddings keep the reads and the transposing writes off shared
+// banks).  It lies behind the epilogue strips inside the drained ring where that has the room (16
+// channels at a time), else behind the tile's operands (8 at a time).
+template <class C>
+struct SideCfg {
+  static constexpr int bytes(int jc) { return (C::kBM * (jc + 1) + (C::kBN + 4) * jc) * 4; }
+  static constexpr int kJC = C::kEpiBytes + bytes(16) <= C::kMainBytes ? 16 : 8;
+  static constexpr int kOff = C::kEpiBytes + bytes(kJC) <= C::kMainBytes ? C::kEpiBytes : (C::kFlagOff + 32 + 15) / 16 * 16;
+  static constexpr int kSmem = kOff + bytes(kJC) > C::kSmemBytes ? kOff + bytes(kJC) : C::kSmemBytes;
+  static_assert(kSmem <= 160 * 1024, "the side term's operands fit in LDS");
+};
+
+// The V25 epilogue of a tile (epi_v25 per element: the same products and sums in the same order).
+// Evaluated element by element from memory, each output waits out 2 ko dependent L2 reads, which
+// was the whole launch (300 x 4608 x 3584 with 16 channels, 256x128 tiles on MI355X: 269 us, of
+// which the product itself is 22).  Here every channel value of the tile is read once into LDS and
+// a lane keeps its four columns of wo for all the rows of the strip it stores, so a side term
+// costs one multiply and one add per channel and output.
+template <class C, int I>
+__device__ __forceinline__ void pp_epilogue_v25(const typename C::Acc& acc, const EpiParams& ep, int m0, int n0, int M,
+                                                int N, int vec_ok, char* smem) {
+  if constexpr (I < C::TM) {
+    using S = SideCfg<C>;
+    constexpr int BM = C::kBM, BN = C::kBN, JC = S::kJC;
+    constexpr int kQuads = C::WTN / 4, kT = 32 * kQuads / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+    const int wm = wave / C::kWN, wn = wave % C::kWN;
+    int32_t* region = (int32_t*)(smem + wave * C::kStripBytes);
+    lsk::pp_stage_strip<C::TN, C::kLdc>(acc[I], region);
+    float* sh = (float*)(smem + S::kOff);
+    float* sw = sh + BM * (JC + 1);
+    const int c4 = lane % kQuads, r0 = lane / kQuads;
+    constexpr int kRowStep = 64 / kQuads;
+    const int nl = wn * C::WTN + c4 * 4, n = n0 + nl;
+    const int ml0 = wm * C::WTM + I * 32 + r0;
+    float side[kT][4];
+#pragma unroll
+    for (int t = 0; t < kT; ++t)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) side[t][k] = 0.0f;
+    for (int jc = 0; jc < ep.ko; jc += JC) {
+      const int jn = ep.ko - jc < JC ? ep.ko - jc : JC;
+      __syncthreads();  // every wave is past its reads of the previous channels
+      for (int i = tid; i < BM * JC; i += C::kThreads) {
+        const int r = i / JC, j = i % JC;
+        sh[r * (JC + 1) + j] = (j < jn && m0 + r < M) ? ep.ho[(int64_t)(m0 + r) * ep.ko + jc + j] : 0.0f;
+      }
+      for (int i = tid; i < BN * JC; i += C::kThreads) {
+        const int c = i / JC, j = i % JC;
+        float v = 0.0f;
+        if (j < jn && n0 + c < N) {
+          const int64_t o = (int64_t)(n0 + c) * ep.ko + jc + j;
+          v = ep.wo_dtype == LSK_BF16 ? bf16_to_f32(((const uint16_t*)ep.wo)[o]) : ((const float*)ep.wo)[o];
+        }
+        sw[j * (BN + 4) + c] = v;
+      }
+      __syncthreads();
+      for (int j = 0; j < jn; ++j) {
+        const v4f w = *(const v4f*)(sw + j * (BN + 4) + nl);
+#pragma unroll
+        for (int t = 0; t < kT; ++t) {
+          const float h = sh[(ml0 + kRowStep * t) * (JC + 1) + j];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) side[t][k] = f32_add(side[t][k], f32_mul(h, w[k]));
+        }
+      }
+    }
+    const float* sc_row = (const float*)(smem + C::kScaleOff);
+    const float* sc_ws = sc_row + BM;
+    const v4f wsq = *(const v4f*)(sc_ws + nl), bq = *(const v4f*)(sc_ws + BN + nl);
+    const bool vec = vec_ok && n + 4 <= N, has_bias = ep.bias != nullptr;
+#pragma unroll
+    for (int t = 0; t < kT; ++t) {
+      const v4i v = *(const v4i*)(region + (r0 + kRowStep * t) * C::kLdc + c4 * 4);
+      const int m = m0 + ml0 + kRowStep * t;
+      const float rv = sc_row[ml0 + kRowStep * t];
+      float y[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        y[k] = bfr(f32_add(bfr(f32_mul(f32_mul((float)v[k], wsq[k]), rv)), side[t][k]));
+        if (has_bias) y[k] = bfr(f32_add(y[k], bq[k]));
+      }
+      if (m >= M || n >= N) continue;
+      const int64_t o = (int64_t)m * ep.ldo + n;
+      if (vec) {
+        store4_out(ep.out, LSK_EPI_V25, ep.out_dtype, o, y, v);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (n + k < N) store_out(ep.out, ep.out_dtype, o + k, y[k]);
+      }
+    }
+    pp_epilogue_v25<C, I + 1>(acc, ep, m0, n0, M, N, vec_ok, smem);
+  }
+}
+
 // One dense tile (eight-wave ping-pong or four-wave main loop, MAIN); same operand contract and
 // tile order as gemm_i8_mfma_kernel.  The epilogue operands of the tile (asc / row exponents,
 // ws, bias, column exponents) are loaded into registers before the main loop and parked in LDS
-// after it, so the epilogue itself touches global memory only to store.
-template <class C, class MAIN>
+// after it, so the epilogue itself touches global memory only to store.  V25 (the outlier epilogue)
+// is an instantiation of its own, so the other orders' kernels keep their registers and code size.
+template <class C, bool V25, class MAIN>
 __device__ __forceinline__ void contract_tile(const int8_t* __restrict__ A, int lda, const int8_t* __restrict__ W,
                                               int ldw, int M, int N, int K, const EpiParams& ep, int vec_ok,
                                               char* smem_pp, MAIN main) {
@@ -317,6 +411,10 @@ __device__ __forceinline__ void contract_tile(const int8_t* __restrict__ A, int 
   if (lane == 0) sc_flag[wave] = wave_odd ? 1 : 0;
   if (kWaves < 8 && tid < 8 - kWaves) sc_flag[kWaves + tid] = 0;
   __syncthreads();
+  if constexpr (V25) {
+    pp_epilogue_v25<C, 0>(acc, ep, m0, n0, M, N, vec_ok, smem_pp);
+    return;
+  }
   // each wave stages its own 32-row strips, then stores them through the epilogue
   const bool bias = ep.bias != nullptr;
   if (ep.order == LSK_EPI_V21 && !bias && vec_ok == 2 && m0 + BM <= M && n0 + BN <= N &&
@@ -355,13 +453,13 @@ __device__ __forceinline__ void contract_tile(const int8_t* __restrict__ A, int 
 }
 
 // Dense ping-pong tile kernel (512 threads, eight waves in two alternating groups).
-template <int BM, int BN, int WM, int WN, int RING, int BKB>
+template <int BM, int BN, int WM, int WN, int RING, int BKB, bool V25>
 __global__ __launch_bounds__(512, (RING == 3 && BKB == 64 ? 2 : 1)) void gemm_i8_pp_kernel(const int8_t* __restrict__ A, int lda,
                                                          const int8_t* __restrict__ W, int ldw, int M, int N, int K,
                                                          EpiParams ep, int vec_ok) {
   using C = lsk::PPCfg<BM, BN, WM, WN, RING, BKB>;
   extern __shared__ __attribute__((aligned(16))) char smem_pp[];
-  contract_tile<C>(A, lda, W, ldw, M, N, K, ep, vec_ok, smem_pp,
+  contract_tile<C, V25>(A, lda, W, ldw, M, N, K, ep, vec_ok, smem_pp,
                    [](typename C::Acc& acc, __amdgpu_buffer_rsrc_t ra, const typename C::RowsA& pa,
                       __amdgpu_buffer_rsrc_t rb, const typename C::RowsB& pb, int K_, char* sm, int pairs) {
                      lsk::pp_mainloop<BM, BN, WM, WN, RING, BKB>(acc, ra, pa, rb, pb, K_, sm, 0, pairs);
@@ -447,13 +545,13 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_pow2_persist_kernel(const i
 }
 
 // Dense four-wave tile kernel (256 threads, one wave per SIMD, 128-row wave tiles; w4_tile.h).
-template <int BM, int BN, int RING>
+template <int BM, int BN, int RING, bool V25>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_i8_w4_kernel(
     const int8_t* __restrict__ A, int lda, const int8_t* __restrict__ W, int ldw, int M, int N, int K, EpiParams ep,
     int vec_ok) {
   using C = lsk::W4Cfg<BM, BN, RING>;
   extern __shared__ __attribute__((aligned(16))) char smem_pp[];
-  contract_tile<C>(A, lda, W, ldw, M, N, K, ep, vec_ok, smem_pp,
+  contract_tile<C, V25>(A, lda, W, ldw, M, N, K, ep, vec_ok, smem_pp,
                    [](typename C::Acc& acc, __amdgpu_buffer_rsrc_t ra, const typename C::RowsA& pa,
                       __amdgpu_buffer_rsrc_t rb, const typename C::RowsB& pb, int K_, char* sm, int) {
                      lsk::w4_mainloop<C>(acc, ra, pa, rb, pb, K_, sm);  // row-major A only
@@ -1407,16 +1505,20 @@ static int launch_tile(const int8_t* a, int lda, const int8_t* w, int ldw, int M
   return check_launch(name);
 }
 
-template <int BM, int BN, int WM, int WN, int RING = 4, int BKB = 64>
+template <int BM, int BN, int WM, int WN, int RING = 4, int BKB = 64, bool V25 = false>
 static int launch_pp(const int8_t* a, int lda, const int8_t* w, int ldw, int M, int N, int K, const EpiParams& ep,
                      int vec_ok, hipStream_t s, const char* name) {
+  if constexpr (!V25)
+    if (ep.order == LSK_EPI_V25)
+      return launch_pp<BM, BN, WM, WN, RING, BKB, true>(a, lda, w, ldw, M, N, K, ep, vec_ok, s, name);
   using C = PPCfg<BM, BN, WM, WN, RING, BKB>;
+  constexpr int kSmem = V25 ? SideCfg<C>::kSmem : C::kSmemBytes;
   static std::atomic<bool> attr_set{false};
-  auto kern = gemm_i8_pp_kernel<BM, BN, WM, WN, RING, BKB>;
+  auto kern = gemm_i8_pp_kernel<BM, BN, WM, WN, RING, BKB, V25>;
   if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::kSmemBytes) !=
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kSmem) !=
         hipSuccess) {
-      set_error("%s: cannot reserve %d bytes of LDS", name, C::kSmemBytes);
+      set_error("%s: cannot reserve %d bytes of LDS", name, kSmem);
       return LSK_ERR_HIP;
     }
     attr_set = true;
@@ -1427,7 +1529,7 @@ static int launch_pp(const int8_t* a, int lda, const int8_t* w, int ldw, int M, 
   // (the kernel's fast epilogue)
   const int64_t esz = (ep.out_dtype == LSK_BF16 || ep.out_dtype == LSK_F16) ? 2 : 4;
   const int vflag = (vec_ok && (int64_t)(BM - 1) * ep.ldo * esz + BN * esz < 0x7fffffff) ? 2 : vec_ok;
-  if constexpr (BM == 256 && BN == 256 && WM == 4 && WN == 2 && RING == 4 && BKB == 64) {
+  if constexpr (!V25 && BM == 256 && BN == 256 && WM == 4 && WN == 2 && RING == 4 && BKB == 64) {
     // whole tiles under POW2 with binary32 out: the persistent kernel, one block per CU
     if (g_pp_persist != 0 && ep.order == LSK_EPI_POW2 && ep.ecol == nullptr && ep.out_dtype == LSK_F32 &&
         vflag == 2 && M % BM == 0 && N % BN == 0 && K % BKB == 0 && K / BKB >= C::kRing + 2) {
@@ -1447,21 +1549,23 @@ static int launch_pp(const int8_t* a, int lda, const int8_t* w, int ldw, int M, 
       return check_launch(name);
     }
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(C::kThreads), C::kSmemBytes, s, a, lda, w, ldw, M, N, K, ep,
-                     vflag);
+  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(C::kThreads), kSmem, s, a, lda, w, ldw, M, N, K, ep, vflag);
   return check_launch(name);
 }
 
-template <int BM, int BN, int RING = 4>
+template <int BM, int BN, int RING = 4, bool V25 = false>
 static int launch_w4(const int8_t* a, int lda, const int8_t* w, int ldw, int M, int N, int K, const EpiParams& ep,
                      int vec_ok, hipStream_t s, const char* name) {
+  if constexpr (!V25)
+    if (ep.order == LSK_EPI_V25) return launch_w4<BM, BN, RING, true>(a, lda, w, ldw, M, N, K, ep, vec_ok, s, name);
   using C = W4Cfg<BM, BN, RING>;
+  constexpr int kSmem = V25 ? SideCfg<C>::kSmem : C::kSmemBytes;
   static std::atomic<bool> attr_set{false};
-  auto kern = gemm_i8_w4_kernel<BM, BN, RING>;
+  auto kern = gemm_i8_w4_kernel<BM, BN, RING, V25>;
   if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::kSmemBytes) !=
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kSmem) !=
         hipSuccess) {
-      set_error("%s: cannot reserve %d bytes of LDS", name, C::kSmemBytes);
+      set_error("%s: cannot reserve %d bytes of LDS", name, kSmem);
       return LSK_ERR_HIP;
     }
     attr_set = true;
@@ -1470,8 +1574,7 @@ static int launch_w4(const int8_t* a, int lda, const int8_t* w, int ldw, int M, 
   LSK_REQUIRE(tiles <= 0x7fffffff, "gemm: too many tiles");
   const int64_t esz = (ep.out_dtype == LSK_BF16 || ep.out_dtype == LSK_F16) ? 2 : 4;
   const int vflag = (vec_ok && (int64_t)(BM - 1) * ep.ldo * esz + BN * esz < 0x7fffffff) ? 2 : vec_ok;
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(C::kThreads), C::kSmemBytes, s, a, lda, w, ldw, M, N, K, ep,
-                     vflag);
+  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(C::kThreads), kSmem, s, a, lda, w, ldw, M, N, K, ep, vflag);
   return check_launch(name);
 }
 

@@ -190,6 +190,19 @@ LSK_DEV uint2 quant8_pack(const float (&v)[8], float s, float r) {
   return make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
 }
 
+// Block-wide max of non-negative floats; every thread gets the result.
+template <int THREADS>
+LSK_DEV float block_max(float v, float* red) {
+  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (lane == 0) red[wave] = v;
+  __syncthreads();
+  float r = red[0];
+  for (int w = 1; w < THREADS / 64; ++w) r = fmaxf(r, red[w]);
+  __syncthreads();
+  return r;
+}
+
 // Load 8 consecutive elements of dtype DT (16-byte aligned) as binary32.
 template <int DT>
 LSK_DEV void load8_as_f32(const void* x, int64_t i8, float* v) {

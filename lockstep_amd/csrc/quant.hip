@@ -16,19 +16,6 @@ bool gemm_takes_skinny(const int8_t* w, int64_t ldw, int64_t M, int64_t N, int64
 
 namespace {
 
-// Block-wide max of non-negative floats; every thread gets the result.
-template <int THREADS>
-LSK_DEV float block_max(float v, float* red) {
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  float r = red[0];
-  for (int w = 1; w < THREADS / 64; ++w) r = fmaxf(r, red[w]);
-  __syncthreads();
-  return r;
-}
-
 // One block per row.  Pass 1: amax over the row (exact, order-free).  Pass 2: quantise.
 // Vector path: 8 elements per thread-step when the row is 16-byte aligned and K % 8 == 0.
 template <int THREADS>
