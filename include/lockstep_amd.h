@@ -223,7 +223,7 @@ int lsk_rmsnorm_float(const void* x, int x_dtype, int64_t ldx, int64_t R, int64_
 int lsk_tree_sum(const float* v, int64_t ldv, int64_t R, int64_t n, float* out, void* stream);
 
 /* Tuning control with no counterpart in the reference: force the dense kernel
- * (0: 128x128 register-staged tile, 4 waves of 64x64; 1: ping-pong 256x256, 8 waves of 64x128;
+ * (0: ping-pong 128x128 with 128-byte K stages, 8 waves of 32x64; 1: ping-pong 256x256, 8 waves of 64x128;
  * 2: ping-pong 256x256, 8 waves of 128x64; 3: ping-pong 256x128, 8 waves of 64x64;
  * 4: ping-pong 128x256, 8 waves of 64x64; 5: the decode GEMV when M <= 32, else tile 0;
  * 6, 7: for M <= 4 the 8-row register-buffered / LDS-ring GEMV instead of the whole-row GEMV;
@@ -234,10 +234,22 @@ int lsk_tree_sum(const float* v, int64_t ldv, int64_t R, int64_t n, float* out, 
  * refused); 18: ping-pong 256x128 with 128-byte K stages
  * in a three-stage ring, the shape's default; 19: for every M <= 32 whose activation rows fit in
  * LDS (M * (ceil(K / 1024) * 1024 + 16) <= 160 KB) the skinny GEMV -- A staged in LDS once per
- * block, weight rows streamed into the MFMA operand, the default for 4 < M <= 32 -- other M as 5)
+ * block, weight rows streamed into the MFMA operand, the default for 4 < M <= 32 -- other M as 5;
+ * 20: ping-pong 64x128 with 128-byte K stages)
  * or -1 to choose by shape (the default).  Results are identical for every choice; only speed differs.
  * The choice applies to the calling host thread's later launches only (thread-local). */
 int lsk_gemm_select(int tile_id);
+
+/* No counterpart in the reference: bytes of room for K-split partial sums with which M rows, N output
+ * channels and depth K are fastest (0 where no split is taken; no device work).  lsk_w8a8_matmul,
+ * lsk_w8a8_outlier_linear and lsk_linear_dyn use whatever their workspace holds past the size their
+ * own workspace query gives, so a caller adds this to it; with less room they split less or not at
+ * all.  The same results. */
+int64_t lsk_gemm_split_bytes(int64_t M, int64_t N, int64_t K);
+
+/* Tuning control with no counterpart in the reference: K slices of the tiles 0 and 20 when selected,
+ * room permitting (0, the default: one).  Results are identical.  Thread-local. */
+int lsk_gemm_split(int n);
 
 /* Tuning control with no counterpart in the reference: the launch shape of the skinny decode GEMV
  * (lsk_gemm_select 19): gpb groups of 16 weight rows per block, kw waves per group splitting K,

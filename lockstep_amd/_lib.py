@@ -54,6 +54,8 @@ SIGNATURES = {
                                _I64, _P, _P, _P]),
     "lsk_tree_sum": (_I, [_P, _I64, _I64, _I64, _P, _P]),
     "lsk_gemm_select": (_I, [_I]),
+    "lsk_gemm_split": (_I, [_I]),
+    "lsk_gemm_split_bytes": (_I64, [_I64, _I64, _I64]),
     "lsk_gemm_skinny_shape": (_I, [_I, _I, _I]),
     "lsk_moe_skinny_shape": (_I, [_I, _I]),
     "lsk_moe_pp_skinny_rows": (_I, [_I]),

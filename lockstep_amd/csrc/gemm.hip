@@ -3,7 +3,8 @@
 //   prefill (M > 128): eight-wave ping-pong MFMA tiles (pp_tile.h), v_mfma_i32_32x32x32_i8,
 //                     four 64-byte K stages in flight through direct-to-LDS loads, XCD-aware
 //                     tile order, epilogue operands staged in LDS.
-//   small   (32 < M <= 128): register-staged 128x128 MFMA tiles (mfma_tile.h).
+//   mid     (M > 16, at most one 128x128 tile per CU): the same main loop on 64x128 and 128x128
+//                     tiles with 128-byte K stages, K split over blocks where the tiles leave CUs idle.
 //   decode  (M <= 32): weight-streaming GEMV on the same MFMA (rows padded to 16 in registers),
 //                     K split over the block's waves and reduced exactly in LDS.
 //   generic:          any stride / alignment / K, one thread per output (correctness path).
@@ -28,70 +29,6 @@
 namespace {
 
 using lsk::zero4;
-
-// Dense tile kernel: C[m, n] = sum_k A[m, k] * W[n, k] with the epilogue applied per element.
-// A and W are K-contiguous with 16-byte aligned rows and K % 16 == 0.  Logical tile ids walk
-// M-fastest inside groups of 16 M-tiles after the XCD remap.
-template <int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_i8_mfma_kernel(
-    const int8_t* __restrict__ A, int lda, const int8_t* __restrict__ W, int ldw, int M, int N, int K,
-    EpiParams ep, int vec_ok) {
-  using C = lsk::TileCfg<BM, BN, WM, WN>;
-  extern __shared__ v4i smem[];
-  const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;
-  const int L = lsk::xcd_logical_id(blockIdx.x, mtiles * ntiles);
-  constexpr int GM = LSK_GROUP_M;
-  const int group = L / (GM * ntiles);
-  const int first_m = group * GM;
-  const int gsize = (mtiles - first_m) < GM ? (mtiles - first_m) : GM;
-  const int r = L - group * GM * ntiles;
-  const int m0 = (first_m + r % gsize) * BM, n0 = (r / gsize) * BN;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
-  const int wm = wave / WN, wn = wave % WN;
-  // resources start at the tile's first row: offsets stay below BM * lda
-  const __amdgpu_buffer_rsrc_t ra_res = lsk::make_rsrc(A + (int64_t)m0 * lda, (int64_t)(M - m0) * lda);
-  const __amdgpu_buffer_rsrc_t rb_res = lsk::make_rsrc(W + (int64_t)n0 * ldw, (int64_t)(N - n0) * ldw);
-  typename C::RowsA pa;
-  typename C::RowsB pb;
-#pragma unroll
-  for (int j = 0; j < C::kAPer; ++j) {
-    int row, c;
-    lsk::chunk_of<C::kThreads>(tid, j, row, c);
-    pa[j] = (m0 + row < M) ? (uint32_t)(row * lda) : lsk::kOob;
-  }
-#pragma unroll
-  for (int j = 0; j < C::kBPer; ++j) {
-    int row, c;
-    lsk::chunk_of<C::kThreads>(tid, j, row, c);
-    pb[j] = (n0 + row < N) ? (uint32_t)(row * ldw) : lsk::kOob;
-  }
-  typename C::Acc acc;
-#pragma unroll
-  for (int i = 0; i < C::TM; ++i)
-#pragma unroll
-    for (int j = 0; j < C::TN; ++j) acc[i][j] = lsk::zero16();
-
-  lsk::mfma_mainloop<BM, BN, WM, WN>(acc, ra_res, pa, rb_res, pb, K, smem);
-
-  int32_t* region = (int32_t*)smem + wave * C::kStripInts;
-  constexpr int kQuads = C::WTN / 4;
-#pragma unroll
-  for (int i = 0; i < C::TM; ++i)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      lsk::stage_half<C::TN, C::kLdc>(acc[i], h, region);
-      __syncthreads();
-      for (int q = lane; q < 16 * kQuads; q += 64) {
-        const int row = q / kQuads, c4 = q - row * kQuads;
-        const v4i v = *(const v4i*)(region + row * C::kLdc + c4 * 4);
-        const int m = m0 + wm * C::WTM + i * 32 + h * 16 + row;
-        const int n = n0 + wn * C::WTN + c4 * 4;
-        if (m < M && n < N) epilogue_store4(ep, m, n, N, v, vec_ok && n + 4 <= N);
-      }
-      __syncthreads();
-    }
-}
 
 // Epilogue of the ping-pong kernel, one staged 32-row strip (strip i of the wave's tile, in the
 // wave's LDS region): the contract epilogue over four consecutive columns per lane (a lane
@@ -327,14 +264,25 @@ __device__ __forceinline__ void pp_epilogue_v25(const typename C::Acc& acc, cons
 // ws, bias, column exponents) are loaded into registers before the main loop and parked in LDS
 // after it, so the epilogue itself touches global memory only to store.  V25 (the outlier epilogue)
 // is an instantiation of its own, so the other orders' kernels keep their registers and code size.
-template <class C, bool V25, class MAIN>
+// kSplit: K in ep.nsplit slices of ep.kslice bytes, blocks of one slice adjacent (an XCD's blocks
+// share its activation columns); a block writes its exact int32 sums to slice ks of ep.part
+// [nsplit][M][N rounded up to 4] and split_combine_kernel adds the slices and applies the epilogue.
+enum TileMode { kPlain = 0, kV25 = 1, kSplit = 2 };
+template <class C, int MODE, class MAIN>
 __device__ __forceinline__ void contract_tile(const int8_t* __restrict__ A, int lda, const int8_t* __restrict__ W,
                                               int ldw, int M, int N, int K, const EpiParams& ep, int vec_ok,
                                               char* smem_pp, MAIN main) {
   constexpr int BM = C::kBM, BN = C::kBN;
   constexpr int kWaves = C::kThreads / 64;
   const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;
-  const int L = lsk::xcd_logical_id(blockIdx.x, mtiles * ntiles);
+  int L = lsk::xcd_logical_id(blockIdx.x, mtiles * ntiles * (MODE == kSplit ? ep.nsplit : 1));
+  int ks = 0, k0 = 0;
+  if constexpr (MODE == kSplit) {
+    ks = L / (mtiles * ntiles);
+    L -= ks * mtiles * ntiles;
+    k0 = ks * ep.kslice;
+    K = K - k0 < ep.kslice ? K - k0 : ep.kslice;
+  }
   constexpr int GM = LSK_GROUP_M;
   const int group = L / (GM * ntiles);
   const int first_m = group * GM;
@@ -347,11 +295,11 @@ __device__ __forceinline__ void contract_tile(const int8_t* __restrict__ A, int 
   // epilogue operands: thread t holds row m0 + t and column n0 + t
   float s_row = 0.0f, s_ws = 0.0f, s_b = 0.0f;
   int s_ec = 0;
-  if (tid < BM && m0 + tid < M) {
+  if (MODE != kSplit && tid < BM && m0 + tid < M) {
     if (ep.order == LSK_EPI_POW2) s_row = __int_as_float(ep.erow ? ep.erow[m0 + tid] : 0);
     else if (ep.order != LSK_EPI_RAW) s_row = ep.asc[m0 + tid];
   }
-  if (tid < BN && n0 + tid < N) {
+  if (MODE != kSplit && tid < BN && n0 + tid < N) {
     if (ep.order == LSK_EPI_POW2) {
       s_ec = ep.ecol ? ep.ecol[n0 + tid] : 0;
     } else if (ep.order != LSK_EPI_RAW) {
@@ -365,8 +313,9 @@ __device__ __forceinline__ void contract_tile(const int8_t* __restrict__ A, int 
   const int ap = ep.pairs & 1, bp = ep.pairs & 2;
   const int64_t a_rows = ap ? (int64_t)((M - m0 + 1) & ~1) : (int64_t)(M - m0);
   const int64_t b_rows = bp ? (int64_t)((N - n0 + 1) & ~1) : (int64_t)(N - n0);
-  const __amdgpu_buffer_rsrc_t ra_res = lsk::make_rsrc(A + (int64_t)m0 * lda, a_rows * lda);
-  const __amdgpu_buffer_rsrc_t rb_res = lsk::make_rsrc(W + (int64_t)n0 * ldw, b_rows * ldw);
+  const int ka0 = ap ? 2 * k0 : k0, kb0 = bp ? 2 * k0 : k0;  // (k0 is a multiple of 64)
+  const __amdgpu_buffer_rsrc_t ra_res = lsk::make_rsrc(A + (int64_t)m0 * lda + ka0, a_rows * lda - ka0);
+  const __amdgpu_buffer_rsrc_t rb_res = lsk::make_rsrc(W + (int64_t)n0 * ldw + kb0, b_rows * ldw - kb0);
   typename C::RowsA pa;
   typename C::RowsB pb;
 #pragma unroll
@@ -391,6 +340,28 @@ __device__ __forceinline__ void contract_tile(const int8_t* __restrict__ A, int 
 
   main(acc, ra_res, pa, rb_res, pb, K, smem_pp, ep.pairs);
 
+  if constexpr (MODE == kSplit) {
+    // straight from the accumulators: register r of lane l holds row 8 (r / 4) + 4 (l / 32) + r % 4,
+    // column l % 32 of each 32 x 32 block, so an instruction stores 128 bytes of two rows
+    const int np = (N + 3) & ~3;
+    const int wm = wave / C::kWN, wn = wave % C::kWN;
+    int32_t* base = ep.part + ((int64_t)ks * M + m0) * np + n0;
+    const __amdgpu_buffer_rsrc_t ro = lsk::make_rsrc((const int8_t*)base, ((int64_t)(M - m0) * np - n0) * 4);
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j) {
+      const int c = wn * C::WTN + j * 32 + (lane & 31);
+      const bool cok = n0 + c < N;
+#pragma unroll
+      for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+          const int row = wm * C::WTM + i * 32 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
+          __builtin_amdgcn_raw_buffer_store_b32((uint32_t)acc[i][j][q], ro,
+                                                cok && m0 + row < M ? (uint32_t)((row * np + c) * 4) : lsk::kOob, 0, 0);
+        }
+    }
+    return;
+  }
   // every wave is past its last read of the LDS ring
   float* sc_row = (float*)(smem_pp + C::kScaleOff);
   float* sc_ws = sc_row + BM;
@@ -411,7 +382,7 @@ __device__ __forceinline__ void contract_tile(const int8_t* __restrict__ A, int 
   if (lane == 0) sc_flag[wave] = wave_odd ? 1 : 0;
   if (kWaves < 8 && tid < 8 - kWaves) sc_flag[kWaves + tid] = 0;
   __syncthreads();
-  if constexpr (V25) {
+  if constexpr (MODE == kV25) {
     pp_epilogue_v25<C, 0>(acc, ep, m0, n0, M, N, vec_ok, smem_pp);
     return;
   }
@@ -453,13 +424,13 @@ __device__ __forceinline__ void contract_tile(const int8_t* __restrict__ A, int 
 }
 
 // Dense ping-pong tile kernel (512 threads, eight waves in two alternating groups).
-template <int BM, int BN, int WM, int WN, int RING, int BKB, bool V25>
+template <int BM, int BN, int WM, int WN, int RING, int BKB, int MODE>
 __global__ __launch_bounds__(512, (RING == 3 && BKB == 64 ? 2 : 1)) void gemm_i8_pp_kernel(const int8_t* __restrict__ A, int lda,
                                                          const int8_t* __restrict__ W, int ldw, int M, int N, int K,
                                                          EpiParams ep, int vec_ok) {
   using C = lsk::PPCfg<BM, BN, WM, WN, RING, BKB>;
   extern __shared__ __attribute__((aligned(16))) char smem_pp[];
-  contract_tile<C, V25>(A, lda, W, ldw, M, N, K, ep, vec_ok, smem_pp,
+  contract_tile<C, MODE>(A, lda, W, ldw, M, N, K, ep, vec_ok, smem_pp,
                    [](typename C::Acc& acc, __amdgpu_buffer_rsrc_t ra, const typename C::RowsA& pa,
                       __amdgpu_buffer_rsrc_t rb, const typename C::RowsB& pb, int K_, char* sm, int pairs) {
                      lsk::pp_mainloop<BM, BN, WM, WN, RING, BKB>(acc, ra, pa, rb, pb, K_, sm, 0, pairs);
@@ -551,7 +522,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     int vec_ok) {
   using C = lsk::W4Cfg<BM, BN, RING>;
   extern __shared__ __attribute__((aligned(16))) char smem_pp[];
-  contract_tile<C, V25>(A, lda, W, ldw, M, N, K, ep, vec_ok, smem_pp,
+  contract_tile<C, V25 ? kV25 : kPlain>(A, lda, W, ldw, M, N, K, ep, vec_ok, smem_pp,
                    [](typename C::Acc& acc, __amdgpu_buffer_rsrc_t ra, const typename C::RowsA& pa,
                       __amdgpu_buffer_rsrc_t rb, const typename C::RowsB& pb, int K_, char* sm, int) {
                      lsk::w4_mainloop<C>(acc, ra, pa, rb, pb, K_, sm);  // row-major A only
@@ -1438,6 +1409,95 @@ __global__ __launch_bounds__(256) void epilogue_apply_kernel(const int32_t* __re
   }
 }
 
+// Adds the int32 slices of a K-split product and applies the epilogue: a block of 256 threads takes
+// kRows rows x 256 columns, a lane four columns of every fourth row.  V25: the side term as in
+// pp_epilogue_v25, 16 channels staged in LDS at a time.
+template <bool V25>
+__global__ __launch_bounds__(256) void split_combine_kernel(const int32_t* __restrict__ part, int M, int N, EpiParams ep,
+                                                            int vec_ok) {
+  constexpr int kR = V25 ? 4 : 1;  // rows per thread
+  constexpr int JC = 16, kLdw = 260;
+  __shared__ __attribute__((aligned(16))) float sw[V25 ? JC * kLdw : 4];
+  __shared__ float sh[V25 ? 4 * kR * (JC + 1) : 1];
+  const int np = (N + 3) & ~3;
+  const int n0 = blockIdx.x * 256, m0 = blockIdx.y * 4 * kR;
+  const int c = (threadIdx.x & 63) * 4, n = n0 + c;
+  const int rq = threadIdx.x >> 6;
+  v4i acc[kR];
+#pragma unroll
+  for (int t = 0; t < kR; ++t) {
+    acc[t] = v4i{0, 0, 0, 0};
+    const int m = m0 + rq + 4 * t;
+    if (m < M && n < N)
+      for (int s = 0; s < ep.nsplit; ++s) acc[t] += *(const v4i*)(part + ((int64_t)s * M + m) * np + n);
+  }
+  const bool vec = vec_ok && n + 4 <= N;
+  if constexpr (!V25) {
+    const int m = m0 + rq;
+    if (m < M && n < N) epilogue_store4(ep, m, n, N, acc[0], vec);
+  } else {
+    float side[kR][4];
+#pragma unroll
+    for (int t = 0; t < kR; ++t)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) side[t][k] = 0.0f;
+    for (int jc = 0; jc < ep.ko; jc += JC) {
+      const int jn = ep.ko - jc < JC ? ep.ko - jc : JC;
+      __syncthreads();
+      for (int i = threadIdx.x; i < 4 * kR * JC; i += 256) {
+        const int r = i / JC, j = i % JC;
+        sh[r * (JC + 1) + j] = (j < jn && m0 + r < M) ? ep.ho[(int64_t)(m0 + r) * ep.ko + jc + j] : 0.0f;
+      }
+      for (int i = threadIdx.x; i < 256 * JC; i += 256) {
+        const int cc = i / JC, j = i % JC;
+        float v = 0.0f;
+        if (j < jn && n0 + cc < N) {
+          const int64_t o = (int64_t)(n0 + cc) * ep.ko + jc + j;
+          v = ep.wo_dtype == LSK_BF16 ? bf16_to_f32(((const uint16_t*)ep.wo)[o]) : ((const float*)ep.wo)[o];
+        }
+        sw[j * kLdw + cc] = v;
+      }
+      __syncthreads();
+      for (int j = 0; j < jn; ++j) {
+        const v4f w = *(const v4f*)(sw + j * kLdw + c);
+#pragma unroll
+        for (int t = 0; t < kR; ++t) {
+          const float h = sh[(rq + 4 * t) * (JC + 1) + j];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) side[t][k] = f32_add(side[t][k], f32_mul(h, w[k]));
+        }
+      }
+    }
+    if (n >= N) return;
+    float wsv[4], bv[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      wsv[k] = n + k < N ? ep.ws[n + k] : 0.0f;
+      bv[k] = ep.bias && n + k < N ? ep.bias[n + k] : 0.0f;
+    }
+#pragma unroll
+    for (int t = 0; t < kR; ++t) {
+      const int m = m0 + rq + 4 * t;
+      if (m >= M) continue;
+      const float rv = ep.asc[m];
+      float y[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        y[k] = bfr(f32_add(bfr(f32_mul(f32_mul((float)acc[t][k], wsv[k]), rv)), side[t][k]));
+        if (ep.bias) y[k] = bfr(f32_add(y[k], bv[k]));
+      }
+      const int64_t o = (int64_t)m * ep.ldo + n;
+      if (vec) {
+        store4_out(ep.out, LSK_EPI_V25, ep.out_dtype, o, y, acc[t]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (n + k < N) store_out(ep.out, ep.out_dtype, o + k, y[k]);
+      }
+    }
+  }
+}
+
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
@@ -1484,37 +1544,16 @@ static int cu_count() {
   return n;
 }
 
-template <int BM, int BN, int WM, int WN>
-static int launch_tile(const int8_t* a, int lda, const int8_t* w, int ldw, int M, int N, int K,
-                       const EpiParams& ep, int vec_ok, hipStream_t s, const char* name) {
-  using C = TileCfg<BM, BN, WM, WN>;
-  static std::atomic<bool> attr_set{false};
-  auto kern = gemm_i8_mfma_kernel<BM, BN, WM, WN>;
-  if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::kSmemBytes) !=
-        hipSuccess) {
-      set_error("%s: cannot reserve %d bytes of LDS", name, C::kSmemBytes);
-      return LSK_ERR_HIP;
-    }
-    attr_set = true;
-  }
-  const int64_t tiles = (int64_t)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  LSK_REQUIRE(tiles <= 0x7fffffff, "gemm: too many tiles");
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(C::kThreads), C::kSmemBytes, s, a, lda, w, ldw, M, N, K, ep,
-                     vec_ok);
-  return check_launch(name);
-}
-
-template <int BM, int BN, int WM, int WN, int RING = 4, int BKB = 64, bool V25 = false>
+template <int BM, int BN, int WM, int WN, int RING = 4, int BKB = 64, int MODE = kPlain>
 static int launch_pp(const int8_t* a, int lda, const int8_t* w, int ldw, int M, int N, int K, const EpiParams& ep,
                      int vec_ok, hipStream_t s, const char* name) {
-  if constexpr (!V25)
+  if constexpr (MODE == kPlain)
     if (ep.order == LSK_EPI_V25)
-      return launch_pp<BM, BN, WM, WN, RING, BKB, true>(a, lda, w, ldw, M, N, K, ep, vec_ok, s, name);
+      return launch_pp<BM, BN, WM, WN, RING, BKB, kV25>(a, lda, w, ldw, M, N, K, ep, vec_ok, s, name);
   using C = PPCfg<BM, BN, WM, WN, RING, BKB>;
-  constexpr int kSmem = V25 ? SideCfg<C>::kSmem : C::kSmemBytes;
+  constexpr int kSmem = MODE == kV25 ? SideCfg<C>::kSmem : C::kSmemBytes;
   static std::atomic<bool> attr_set{false};
-  auto kern = gemm_i8_pp_kernel<BM, BN, WM, WN, RING, BKB, V25>;
+  auto kern = gemm_i8_pp_kernel<BM, BN, WM, WN, RING, BKB, MODE>;
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kSmem) !=
         hipSuccess) {
@@ -1523,13 +1562,13 @@ static int launch_pp(const int8_t* a, int lda, const int8_t* w, int ldw, int M, 
     }
     attr_set = true;
   }
-  const int64_t tiles = (int64_t)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  const int64_t tiles = (int64_t)((M + BM - 1) / BM) * ((N + BN - 1) / BN) * (MODE == kSplit ? ep.nsplit : 1);
   LSK_REQUIRE(tiles <= 0x7fffffff, "gemm: too many tiles");
   // 2: vector stores allowed and a whole tile's output span addressable by 32-bit offsets
   // (the kernel's fast epilogue)
   const int64_t esz = (ep.out_dtype == LSK_BF16 || ep.out_dtype == LSK_F16) ? 2 : 4;
   const int vflag = (vec_ok && (int64_t)(BM - 1) * ep.ldo * esz + BN * esz < 0x7fffffff) ? 2 : vec_ok;
-  if constexpr (!V25 && BM == 256 && BN == 256 && WM == 4 && WN == 2 && RING == 4 && BKB == 64) {
+  if constexpr (MODE == kPlain && BM == 256 && BN == 256 && WM == 4 && WN == 2 && RING == 4 && BKB == 64) {
     // whole tiles under POW2 with binary32 out: the persistent kernel, one block per CU
     if (g_pp_persist != 0 && ep.order == LSK_EPI_POW2 && ep.ecol == nullptr && ep.out_dtype == LSK_F32 &&
         vflag == 2 && M % BM == 0 && N % BN == 0 && K % BKB == 0 && K / BKB >= C::kRing + 2) {
@@ -1580,7 +1619,13 @@ static int launch_w4(const int8_t* a, int lda, const int8_t* w, int ldw, int M, 
 
 static int pick_tile(int64_t M, int64_t N) {
   if (g_force_tile >= 0) return g_force_tile;
-  if (M <= 128) return 0;  // few rows: the 128x128 register-staged tile wastes least
+  // up to 128 rows of a weight with more than 256 128-column tiles (mid_plan takes the others):
+  // 256 columns a tile (MI355X, 37888 x 3584, M = 72: 47.1 us against 49.4 on 128x128 tiles in two rounds)
+  if (M <= 128) return 4;
+  // at most one 128x128 tile per CU, left by mid_plan for a K of under eight stages, where no split
+  // pays and the tile reads either layout (MI355X, us, 256x128 / 128x128: 768 x 512 at M = 512 10.8 /
+  // 9.1, 4096 x 896 at M = 200 / 1000 15.0 / 11.1 and 17.1 / 13.7)
+  if (M <= 2048 && (M + 127) / 128 * ((N + 127) / 128) <= 256) return 0;
   // Ping-pong tiles: whole rounds of 256 blocks (one per CU) are what a launch costs.  A
   // 256x128 tile takes 0.68 of a 256x256 tile's time (measured on MI355X at the Llama-3.1-8B /
   // Qwen2.5-7B prefill shapes), so pick the shape with the smaller rounds x tile cost.  The
@@ -1889,6 +1934,69 @@ int launch_gemv_rowq(const void* x, int x_dtype, const int8_t* w, int ldw, int N
 #undef LSK_RQ
 }
 
+// K slices of a forced 64x128 / 128x128 tile (lsk_gemm_split: 0 one).
+thread_local int g_split = 0;
+
+static int64_t split_bytes(int64_t M, int64_t N, int S) { return S > 1 ? S * M * ((N + 3) / 4 * 4) * 4 : 0; }
+
+// One launch of 64x128 (rows64) or 128x128 tiles, K in S slices; with S > 1 the sums go through
+// ep.part and split_combine_kernel.
+static int launch_mid(bool rows64, int S, const int8_t* a, int lda, const int8_t* w, int ldw, int M, int N, int K,
+                      EpiParams ep, hipStream_t s) {
+  const int vec_ok = out_vec_ok(ep.out, ep.out_dtype, ep.ldo) ? 1 : 0;
+  const int stages = (K + 127) / 128, per = (stages + S - 1) / S;
+  ep.nsplit = (stages + per - 1) / per;
+  ep.kslice = per * 128;
+  if (ep.nsplit <= 1)
+    return rows64 ? launch_pp<64, 128, 2, 4, 5, 128>(a, lda, w, ldw, M, N, K, ep, vec_ok, s, "gemm_i8_pp<64x128,2x4,r5,k128>")
+                  : launch_pp<128, 128, 4, 2, 4, 128>(a, lda, w, ldw, M, N, K, ep, vec_ok, s,
+                                                      "gemm_i8_pp<128x128,4x2,r4,k128>");
+  const int rc = rows64 ? launch_pp<64, 128, 2, 4, 5, 128, kSplit>(a, lda, w, ldw, M, N, K, ep, vec_ok, s,
+                                                                   "gemm_i8_pp<64x128,2x4,r5,k128,split>")
+                        : launch_pp<128, 128, 4, 2, 4, 128, kSplit>(a, lda, w, ldw, M, N, K, ep, vec_ok, s,
+                                                                    "gemm_i8_pp<128x128,4x2,r4,k128,split>");
+  if (rc) return rc;
+  const bool v25 = ep.order == LSK_EPI_V25;
+  const dim3 grid((N + 255) / 256, (M + (v25 ? 15 : 3)) / (v25 ? 16 : 4));
+  if (v25) hipLaunchKernelGGL(split_combine_kernel<true>, grid, dim3(256), 0, s, ep.part, M, N, ep, vec_ok);
+  else hipLaunchKernelGGL(split_combine_kernel<false>, grid, dim3(256), 0, s, ep.part, M, N, ep, vec_ok);
+  return check_launch("split_combine_kernel");
+}
+
+// The mid launch of (M, N, K) with room for part_bytes of partial sums: S = 0 where another kernel
+// is taken.  A 128x128 tile per CU at most (beyond that the 256-row tiles fill the part), more than
+// 16 rows (up to there the GEMVs are ahead) and at most the 2048 the line was fitted on, and up to 32 rows only a weight of 15 M bytes and more
+// that the skinny GEMV leaves and a K split that fits (MI355X, whole call on weights out of cache,
+// us, GEMV / mid: 3584 x 3584 at M = 24 12.5 / 14.9, 4608 x 3584 17.5 / 15.4, 4096 x 14336 28.6 /
+// 23.8, 16000 x 4096 20.4 / 23.2 the skinny GEMV).  Among the tiles and slice counts of at most one
+// block per CU the cheapest by a line through the measured launches: 0.38 (64 rows) or 0.45 us per
+// 128-byte K stage of a block, and for a split 4.5 us plus 8 bytes per partial sum at 6 TB/s.
+// (Before, with 128x128 register-staged tiles up to M = 128 and the 256-row tiles beyond, and after:
+// 3584 x 18944 at M = 72 / 300 / 500 151.7 / 107.2 / 124.9 -> 29.9 / 48.6 / 66.0; 4608 x 3584 at M =
+// 72 / 777 44.4 / 32.7 -> 17.3 / 28.0; 28672 x 4096 at M = 72 58.0 -> 37.7.)
+struct MidPlan {
+  bool rows64;
+  int S;
+};
+static MidPlan mid_plan(int64_t M, int64_t N, int64_t K, int64_t part_bytes) {
+  MidPlan p{false, 0};
+  if (M <= 16 || M > 2048 || (M > 128 && K < 1024) || (M + 127) / 128 * ((N + 127) / 128) > 256) return p;
+  const bool gemv = M <= 32;
+  if (gemv && (N * K < (15 << 20) || gemv_takes_skinny(M, N, K))) return p;
+  const int64_t stages = (K + 127) / 128;
+  double best = 1e30;
+  for (int r64 = M <= 256 ? 1 : 0; r64 >= 0; --r64) {
+    const int64_t t = (M + (r64 ? 63 : 127)) / (r64 ? 64 : 128) * ((N + 127) / 128);
+    for (int S = 1; S == 1 || (S <= 16 && t * S <= 256 && stages >= 4 * S && split_bytes(M, N, S) <= part_bytes); ++S) {
+      const double us = (r64 ? 0.38 : 0.45) * (double)((stages + S - 1) / S) * (double)((t * S + 255) / 256) +
+                        (S > 1 ? 4.5 + 8e-6 / 6 * (double)(S * M * N) : 0.0);
+      if (us < best) best = us, p.rows64 = r64 != 0, p.S = S;
+    }
+  }
+  if (gemv && p.S == 1) p.S = 0;
+  return p;
+}
+
 static bool tiles_fast(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, int64_t M, int64_t N, int64_t K) {
   // the tile kernels address rows by 32-bit offsets inside a 256-row tile
   return (K % 16 == 0) && (lda % 16 == 0) && (ldw % 16 == 0) && aligned16(a) && aligned16(w) && M <= 0x7fffffff &&
@@ -1907,9 +2015,10 @@ bool gemm_takes_skinny(const int8_t* w, int64_t ldw, int64_t M, int64_t N, int64
 bool gemm_takes_pp(const int8_t* w, int64_t ldw, int64_t M, int64_t N, int64_t K, int64_t lda) {
   if (M <= 0 || N <= 0 || !tiles_fast(w, lda, w, ldw, M, N, K)) return false;  // (A aligned: the caller)
   if (M <= 32 && (g_force_tile < 0 || g_force_tile == 5)) return false;
+  if (g_force_tile < 0 && mid_plan(M, N, K, 0).S > 0) return false;  // (row-major: whole lines per K stage)
   if (g_force_tile < 0 && split_columns(M, N) > 0) return true;
   const int t = pick_tile(M, N);
-  return t == 1 || t == 2 || t == 3 || t == 4 || t == 12 || t == 13 || t == 18;
+  return (t == 0 && g_force_tile < 0) || t == 1 || t == 2 || t == 3 || t == 4 || t == 12 || t == 13 || t == 18;
 }
 
 int launch_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, int64_t M, int64_t N, int64_t K,
@@ -1930,6 +2039,14 @@ int launch_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, int6
     return check_launch("gemm_i8_generic_kernel");
   }
   const int iM = (int)M, iN = (int)N, iK = (int)K;
+  if (g_force_tile == 0 || g_force_tile == 20) {
+    const bool fits = g_split > 1 && M <= (1 << 17) && N <= (1 << 21) && split_bytes(M, N, g_split) <= ep.part_bytes;
+    return launch_mid(g_force_tile == 20, fits ? g_split : 1, a, (int)lda, w, (int)ldw, iM, iN, iK, ep, s);
+  }
+  if (g_force_tile < 0 && ep.pairs == 0) {
+    const MidPlan p = mid_plan(M, N, K, ep.part_bytes);
+    if (p.S > 0) return launch_mid(p.rows64, p.S, a, (int)lda, w, (int)ldw, iM, iN, iK, ep, s);
+  }
   if (M <= 32 && (g_force_tile < 0 || g_force_tile == 5)) {
     if (!epi_raw_fits(M, N)) {  // (the GEMVs address their epilogue operands by 32-bit offsets)
       hipLaunchKernelGGL(gemm_i8_generic_kernel, dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, s, a, lda, w,
@@ -1960,7 +2077,7 @@ int launch_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, int6
     case 17: return launch_w4<256, 128>(a, ilda, w, ildw, iM, iN, iK, ep, vec_ok, s, "gemm_i8_w4<256x128>");
     case 18: return launch_pp<256, 128, 4, 2, 3, 128>(a, ilda, w, ildw, iM, iN, iK, ep, vec_ok, s,
                                                       "gemm_i8_pp<256x128,4x2,r3,k128>");
-    default: return launch_tile<128, 128, 2, 2>(a, ilda, w, ildw, iM, iN, iK, ep, vec_ok, s, "gemm_i8<128x128,2x2>");
+    default: return launch_mid(false, 1, a, ilda, w, ildw, iM, iN, iK, ep, s);  // (0; 5 with more than 32 rows)
   }
 }
 
@@ -2031,6 +2148,8 @@ extern "C" int lsk_w8a8_matmul_pairs(const void* x, int x_dtype, int64_t ldx, in
     EpiParams ep{order, out_dtype, ws, nullptr, bias, nullptr, nullptr, 0, out, ldo};
     return lsk::launch_gemv_rowq(x, x_dtype, w, (int)ldw, (int)N, (int)K, ep, (hipStream_t)stream);
   }
+  int32_t* part = (int32_t*)((char*)workspace + need);
+  const int64_t part_bytes = workspace_bytes - need;
   // the row-pair layout when every tile of the GEMM is a ping-pong tile; row-major otherwise
   const int64_t kp = (K + 63) / 64 * 64;
   const bool pair = lsk::rowquant_pair_ok(x, x_dtype, ldx, K) && lsk::gemm_takes_pp(w, ldw, M, N, K, kp);
@@ -2045,11 +2164,16 @@ extern "C" int lsk_w8a8_matmul_pairs(const void* x, int x_dtype, int64_t ldx, in
     ep.pairs = 2;
     return lsk::launch_gemm(q, ldq, w_pairs, kp, M, N, K, ep, (hipStream_t)stream);
   }
-  if (!pair)
-    return (rc = lsk_rowquant(x, x_dtype, M, K, ldx, q, ldq, asc, stream))
-               ? rc
-               : lsk_gemm_w8a8(q, ldq, w, ldw, M, N, K, order, asc, ws, bias, nullptr, nullptr, 0, out, out_dtype,
-                               ldo, stream);
+  if (!pair) {
+    if ((rc = lsk_rowquant(x, x_dtype, M, K, ldx, q, ldq, asc, stream))) return rc;
+    LSK_REQUIRE(K <= 133144, "lsk_w8a8_matmul: K=%lld exceeds the int32-exact bound 133144", (long long)K);
+    LSK_REQUIRE(out && (w || K == 0), "lsk_w8a8_matmul: null pointer");
+    LSK_REQUIRE(ldw >= K && ldo >= N, "lsk_w8a8_matmul: leading dimension too small");
+    EpiParams ep{order, out_dtype, ws, asc, bias, nullptr, nullptr, 0, out, ldo};
+    ep.part = part;
+    ep.part_bytes = part_bytes;
+    return lsk::launch_gemm(q, ldq, w, ldw, M, N, K, ep, (hipStream_t)stream);
+  }
   LSK_REQUIRE(x && w && out && ldw >= K && ldo >= N, "lsk_w8a8_matmul: bad operand");
   if ((rc = lsk::rowquant_pair(x, x_dtype, M, K, ldx, q, ldq, asc, (hipStream_t)stream))) return rc;
   EpiParams ep{order, out_dtype, ws, asc, bias, nullptr, nullptr, 0, out, ldo};
@@ -2105,11 +2229,23 @@ extern "C" int lsk_gemm_persist(int blocks) {
 }
 
 extern "C" int lsk_gemm_select(int tile_id) {
-  LSK_REQUIRE(tile_id >= -1 && tile_id <= 19 && tile_id != 16,
-              "lsk_gemm_select: tile id %d not in [-1, 19] (16, the four-wave 256x256 tile, was removed)", tile_id);
+  LSK_REQUIRE(tile_id >= -1 && tile_id <= 20 && tile_id != 16,
+              "lsk_gemm_select: tile id %d not in [-1, 20] (16, the four-wave 256x256 tile, was removed)", tile_id);
   lsk::g_force_tile = ((tile_id >= 6 && tile_id <= 11) || tile_id == 14 || tile_id == 15 || tile_id == 19) ? 5 : tile_id;
   lsk::g_gemv_mid = tile_id == 14 ? 1 : (tile_id == 15 ? 2 : (tile_id == 19 ? 3 : 0));
   lsk::g_gemv_variant = (tile_id == 6 || tile_id == 7) ? tile_id - 5 : 0;
   lsk::g_row_rpw = (tile_id >= 8 && tile_id <= 11) ? (1 << (tile_id - 8)) : 0;
+  return LSK_OK;
+}
+
+extern "C" int64_t lsk_gemm_split_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 16 != 0) return 0;
+  if (lsk::g_force_tile == 0 || lsk::g_force_tile == 20) return lsk::split_bytes(M, N, lsk::g_split);
+  return lsk::g_force_tile < 0 ? lsk::split_bytes(M, N, lsk::mid_plan(M, N, K, INT64_MAX).S) : 0;
+}
+
+extern "C" int lsk_gemm_split(int n) {
+  LSK_REQUIRE(n >= 0 && n <= 64, "lsk_gemm_split: %d slices not in [0, 64]", n);
+  lsk::g_split = n;
   return LSK_OK;
 }

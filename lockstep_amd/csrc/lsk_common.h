@@ -296,6 +296,11 @@ struct EpiParams {
   // layout -- row pairs interleaved by 64-byte K chunks, element (m, k) at byte (m >> 1) * 2 ld +
   // (k >> 6) * 128 + (m & 1) * 64 + (k & 63), ld % 64 == 0 -- instead of rows of ld bytes
   int pairs = 0;
+  // a caller's room for K-split partial sums (bytes; 16-byte aligned), and the split launch_gemm
+  // chose: nsplit slices of kslice bytes of K
+  int32_t* part = nullptr;
+  int64_t part_bytes = 0;
+  int nsplit = 1, kslice = 0;
 };
 
 // The v2.5 side term of output (m, n) (lockstep_fullstack.py:549-557): sequential in j from +0,

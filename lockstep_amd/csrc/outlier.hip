@@ -296,6 +296,8 @@ extern "C" int lsk_w8a8_outlier_linear(const void* x, int x_dtype, int64_t ldx, 
     ep.ko = (int)ko;
     ep.wo_dtype = wo_dtype;
     ep.pairs = pair;
+    ep.part = (int32_t*)((char*)workspace + need);
+    ep.part_bytes = workspace_bytes - need;
     return lsk::launch_gemm(q, ld, w, ldw, M, N, K, ep, (hipStream_t)stream);
   }
   if ((rc = lsk_outlier_split(x, x_dtype, ldx, M, K, oidx, ko, xm, K, ho, stream))) return rc;

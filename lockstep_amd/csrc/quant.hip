@@ -788,6 +788,8 @@ extern "C" int lsk_linear_dyn(const float* x, int64_t M, int64_t K, int64_t ldx,
   if (!(stages & 2) || M == 0 || N == 0) return LSK_OK;
   EpiParams ep{LSK_EPI_POW2, LSK_F32, nullptr, nullptr, nullptr, erow, nullptr, ew, y, ldy};
   ep.pairs = pair ? 1 : 0;
+  ep.part = (int32_t*)(ws + l.bytes);
+  ep.part_bytes = workspace_bytes - l.bytes;
   // the weight's row-pair copy with the quantised rows' row-pair layout
   if (pair && w_pairs && lsk::gemm_takes_pp(w_pairs, kp, M, N, K, kp)) {
     ep.pairs = 3;

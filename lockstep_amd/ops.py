@@ -112,7 +112,8 @@ def w8a8_matmul(x2: torch.Tensor, w_nk: torch.Tensor, ws: torch.Tensor, bias, or
     out = torch.empty((M, N), dtype=tdt, device=x2.device)
     if M == 0 or N == 0:
         return out
-    nbytes = L.load().lsk_w8a8_matmul_workspace(M, K)
+    lib = L.load()
+    nbytes = lib.lsk_w8a8_matmul_workspace(M, K) + lib.lsk_gemm_split_bytes(M, N, K)
     ws_buf = torch.empty((nbytes,), dtype=torch.uint8, device=x2.device)
     ws, bias = _f32(ws), _f32(bias)
     L.call("lsk_w8a8_matmul_pairs", L.ptr(x2), L.dtype_code(x2.dtype), x2.stride(0) if M > 1 else max(K, 1), M, K,
@@ -164,7 +165,8 @@ def w8a8_outlier_linear(x2: torch.Tensor, oidx: torch.Tensor, wo: torch.Tensor, 
     out = torch.empty((M, N), dtype=_OUT_T[out_dtype], device=x2.device)
     if M == 0 or N == 0:
         return out
-    nbytes = L.load().lsk_w8a8_outlier_linear_workspace(M, K, ko)
+    lib = L.load()
+    nbytes = lib.lsk_w8a8_outlier_linear_workspace(M, K, ko) + lib.lsk_gemm_split_bytes(M, N, K)
     work = torch.empty((nbytes,), dtype=torch.uint8, device=x2.device)
     ws, bias = _f32(ws), _f32(bias)
     L.call("lsk_w8a8_outlier_linear", L.ptr(x2), xc, x2.stride(0) if M > 1 else max(K, 1), M, K, L.ptr(oi), ko,
@@ -381,7 +383,7 @@ def linear_dyn(x: torch.Tensor, w_nk: torch.Tensor, ew: int, stages: int = 3, wo
         ex = torch.empty((1,), dtype=torch.int32, device=x.device)
     nbytes = L.load().lsk_linear_dyn_workspace(M, K)
     if work is None:
-        work = torch.empty((nbytes,), dtype=torch.uint8, device=x.device)
+        work = torch.empty((nbytes + L.load().lsk_gemm_split_bytes(M, N, K),), dtype=torch.uint8, device=x.device)
     elif work.numel() < nbytes:
         raise ValueError("linear_dyn: work buffer of %d bytes, %d needed" % (work.numel(), nbytes))
     if w_pairs is not None and (w_pairs.dtype != torch.int8 or w_pairs.device != x.device

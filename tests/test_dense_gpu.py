@@ -652,3 +652,38 @@ def test_mfma_bf16_acc_probe_exact_cases():
     torch.cuda.synchronize()
     want = (np.einsum("nmk,njk->nmj", a.astype(np.float64), b.astype(np.float64)) + c).astype(np.float32)
     assert np.array_equal(f32_bits(d.cpu().numpy()), f32_bits(want))
+
+
+@pytest.mark.parametrize("tile,split", [(0, 0), (0, 2), (0, 5), (20, 0), (20, 3), (20, 16), (-1, 0)])
+@pytest.mark.parametrize("M,N,K", [(17, 4096, 4096), (64, 130, 2064), (65, 129, 1040), (129, 1001, 2048),
+                                   (33, 2, 144), (300, 516, 3200), (1, 127, 640)])
+def test_k_split_tiles(tile, split, M, N, K):
+    """The 64x128 and 128x128 tiles with K in slices (more slices than stages, a ragged last slice,
+    K past a 128-byte stage, N % 4 != 0): every epilogue the slices are combined under, with the room
+    lsk_gemm_split_bytes asks for, and with none (one slice, the same bits)."""
+    import lockstep_amd._lib as L
+    from lockstep_amd import lockstep_fullstack as FS
+    from lockstep_amd import ref_block_v1 as RB
+    say("k split", tile, split, M, N, K)
+    r = _rng(M + 3 * N + 7 * K)
+    x = (r.standard_normal((M, K)) * 2).astype(F32)
+    W8 = r.integers(-127, 128, (N, K), dtype=np.int8)
+    ws = r.uniform(1e-3, 1e-2, N).astype(F32)
+    bias = (r.standard_normal(N) * 0.1).astype(F32)
+    xd, wd, sd, bd = to_dev(x), to_dev(W8), to_dev(ws), to_dev(bias)
+    L.call("lsk_gemm_select", tile)
+    L.call("lsk_gemm_split", split)
+    try:
+        y = FS.w8a8_matmul(xd, wd, sd, bd, out_dtype=torch.bfloat16)
+        y32 = FS.w8a8_matmul(xd, wd, sd, out_dtype=torch.float32)
+        yp, ex = RB.linear_dyn(xd, wd.t(), 7)
+        acc = FS._int_mm_exact(to_dev(C.rowquant(x)[0]), wd.t())       # no room: one slice
+    finally:
+        L.call("lsk_gemm_select", -1)
+        L.call("lsk_gemm_split", 0)
+    assert np.array_equal(bits(y), C.w8a8_matmul(x, W8, ws, bias, "bf16"))
+    assert np.array_equal(bits(y32), f32_bits(C.w8a8_matmul(x, W8, ws, None, "f32")))
+    q, e = C.quant8_dyn(x)
+    assert int(ex.item()) == e
+    assert np.array_equal(bits(yp), f32_bits((C.gemm_int(q, W8.T).astype(F32) * F32(2.0 ** (-e - 7))).astype(F32)))
+    assert np.array_equal(bits(acc), C.int_mm(C.rowquant(x)[0], W8.T))

@@ -141,7 +141,7 @@ def test_outlier_linear_negative_index_and_empty():
     assert np.array_equal(bits(y3).reshape(6, 128), C.w8a8_outlier_linear(x, oidx, wo, W8, ws, None, "bf16"))
 
 
-@pytest.mark.parametrize("tile", [-1, 1, 2, 3, 4, 12, 13, 17, 18])
+@pytest.mark.parametrize("tile", [-1, 0, 1, 2, 3, 4, 12, 13, 17, 18, 20])
 @pytest.mark.parametrize("M,N,K,ko", [(300, 516, 768, 17), (257, 130, 256, 33), (65, 259, 520, 8), (2, 300, 1000, 5)])
 def test_outlier_tile_epilogues(tile, M, N, K, ko):
     """The side term read from LDS in every tile shape, channel counts below, at and past the 8 or
@@ -154,9 +154,11 @@ def test_outlier_tile_epilogues(tile, M, N, K, ko):
     oidx[-1] = oidx[0]                         # a channel declared twice is masked once, summed twice
     rot = K % 256 == 0
     L.call("lsk_gemm_select", tile)
+    L.call("lsk_gemm_split", 2)                # tiles 0 and 20: the side term added to combined K slices
     try:
         y = FS.w8a8_outlier_linear(bf16_dev(x), to_dev(oidx), bf16_dev(wo), to_dev(W8), to_dev(ws), to_dev(bias),
                                    out_dtype=torch.bfloat16, rot=rot)
     finally:
         L.call("lsk_gemm_select", -1)
+        L.call("lsk_gemm_split", 0)
     assert np.array_equal(bits(y), C.w8a8_outlier_linear(x, oidx, wo, W8, ws, bias, "bf16", rot=rot))
