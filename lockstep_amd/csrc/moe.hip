@@ -24,7 +24,6 @@
 
 namespace {
 
-constexpr float kAmaxFloor = 0x1.5798eep-27f;  // fl32(1e-8)
 constexpr int kBM = lsk::kMoeBM;
 constexpr int kBM2 = 256;  // rows per tile of the 256 x 256 expert tiles (their own tile table)
 thread_local int g_moe_force = -1;  // tuning control: -1 by size, 0 register-staged tile, 1 ping-pong tile, 2 GEMV,
@@ -2761,6 +2760,14 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
   // the experts' row-pair weight copies on the same tiles, when the caller has them
   const bool pair_w = !mx && moe_reads_pair_weights(T, k, E, H, I, rb) && a->w13_pair_ptrs && a->w2_pair_ptrs;
 
+  // MXFP4 experts with per-row scales past the skinny GEMM: six-bit activation planes on the
+  // block-scaled MFMA tiles, for exponent bytes they take (mx6_tile.h).  GPT-OSS-20B on MI355X, bf16
+  // tiles / these: T = 600 gate/up 293 / 213 us, down 163 / 113; T = 4096 850 / 660 and 380 / 320
+  const bool use_mx6 = mx == 1 && T > 256 && !use_mx_skinny && !use_mx_gemv && !a->mx_safe && lsk::mx_variant() == 0 &&
+                       std::min(a->kw13_min, a->kw2_min) >= 16 && std::max(a->kw13_max, a->kw2_max) < 240 &&
+                       ((uintptr_t)a->x & 15) == 0 && a->act_tab && ((uintptr_t)a->act_tab & 15) == 0 &&
+                       R * H * 2 < 0x7fffffff;
+  const int mx6 = std::max(a->kw13_max, a->kw2_max) <= 180 ? 2 : 1;
   // up to 256 tokens: the dispatch and the row quant of x in one launch
   const bool prep_decode = T <= 256 && rb == 0 && mx != 2;
   // routing from logits: inside that launch for up to 4 tokens (a wave per token in its
@@ -2811,6 +2818,8 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
     rc = lsk_rowquant(w.xrot, LSK_F32, T, H, H, w.qx, H, w.ascx, stream);
   } else if (mx == 2) {
     rc = LSK_OK;  // after the dispatch, which clears the flag words it raises
+  } else if (use_mx6) {
+    rc = lsk::launch_rowquant_mx6(a->x, T, H, (uint8_t*)w.qx, w.ascx, s);
   } else if (mx) {
     rc = lsk::launch_rowquant_bf16(a->x, T, H, (uint16_t*)w.qx, w.ascx, s);
   } else {
@@ -2884,6 +2893,11 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
   g1.h = w.h;
   g1.h_amax = w.h_amax;
   g1.lds = a->lds13;
+  if (use_mx6) {
+    g1.mx6 = mx6;
+    g1.lda = H / 32 * 48;
+    g1.a_bytes = T * g1.lda;
+  }
   if (mx == 2) {
     g1.a_scale = nullptr;
     g1.row_flag = w.flagx;
@@ -3004,6 +3018,8 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
     if ((rc = lsk::launch_blockquant_mx2(w.h, I, R, w.offs + E, (int)I, (uint16_t*)w.qh, w.kah, w.flagh, anyf + 1,
                                          use_mx2_gemv ? 1 : lo2, use_mx2_gemv ? 0 : hi2, s)))
       return rc;
+  } else if (use_mx6) {
+    if ((rc = lsk::launch_requant_mx6(w.h, w.h_amax, w.offs + E, R, (int)I, (uint8_t*)w.qh, w.asch, s))) return rc;
   } else if (mx) {
     if ((rc = lsk::launch_requant_bf16(w.h, w.h_amax, w.offs + E, R, (int)I, (uint16_t*)w.qh, w.asch, s))) return rc;
   } else {
@@ -3033,6 +3049,12 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
   g2.row_dst = w.row_dst;
   g2.y = w.slots;
   g2.lds = a->lds2;
+  if (use_mx6) {
+    g2.mx6 = mx6;
+    g2.y_bytes = R * H * 2;
+    g2.lda = I / 32 * 48;
+    g2.a_bytes = R * g2.lda;
+  }
   if (mx == 2) {
     g2.a_scale = nullptr;
     g2.row_flag = w.flagh;

@@ -34,6 +34,10 @@ struct MoeGemmArgs {
   // block-scaled activations (MXFP4 experts, moe_forward_mx2): 0 off; 1 the fused-update kernel
   // over tiles without a flagged row; 2 the general kernel over tiles with one
   int mx2;
+  // MXFP4 experts, per-row scales: A rows as six-bit planes (lda bytes a row), the block-scaled
+  // MFMA tiles (mx6_tile.h); 2: the E8M0 bytes bound the accumulators (kMx6QuietKexp)
+  int mx6;
+  int64_t y_bytes;          // bytes of y (mx6)
   const int32_t* row_flag;  // per A row (gate/up: per token)
   const int32_t* any_flag;  // nonzero when some row is flagged
   const int32_t* a_ka;      // block exponents of the A rows [rows, K/32]
@@ -88,6 +92,11 @@ int64_t mx_skinny_bytes(int64_t rows, int64_t K);
 
 // Row quant emitting the int8 values as bf16 (the MX GEMM's operand form).
 int launch_rowquant_bf16(const uint16_t* x, int64_t T, int64_t H, uint16_t* q, float* asc, hipStream_t s);
+
+// The row quants as six-bit planes (mx6_tile.h; 48 bytes per 32 values, 16-byte aligned rows).
+int launch_rowquant_mx6(const uint16_t* x, int64_t T, int64_t H, uint8_t* q, float* asc, hipStream_t s);
+int launch_requant_mx6(const uint16_t* h, const uint32_t* amax, const int32_t* nrows, int64_t R, int I, uint8_t* q,
+                       float* asc, hipStream_t s);
 
 // Block quant of bf16 rows for block-scaled activations: dequantised bf16 values (integer values
 // on flagged rows), exponents [R, K/32] and row flags (exponent outside [lo, hi]); *any is raised

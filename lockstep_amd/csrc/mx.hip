@@ -5,12 +5,12 @@
 #include "contract_act.h"
 #include "moe_internal.h"
 #include "moe_route.h"
+#include "mx6_tile.h"
 #include "mx_pp.h"
 #include "mx_tile.h"
 
 namespace {
 
-constexpr float kAmaxFloor = 0x1.5798eep-27f;  // fl32(1e-8)
 constexpr int NB = 2;                          // MX blocks per LDS stage (K = 64)
 using Cfg = lsk::MxCfg<128, 128, 2, 2, NB>;
 
@@ -64,6 +64,83 @@ __global__ __launch_bounds__(256) void requant_bf16_kernel(const uint16_t* __res
       o[j] = (uint32_t)q_bf16(bf16_to_f32((uint16_t)(wd[j] & 0xffff)), s, rs) |
              ((uint32_t)q_bf16(bf16_to_f32((uint16_t)(wd[j] >> 16)), s, rs) << 16);
     store16_split(q + p * I + c * 8, o[0], o[1], o[2], o[3]);
+  }
+}
+
+// ---------------------------------------------------------------- quantisers emitting six-bit planes
+// 32 int8 values as the two E2M3 planes of a block (48 bytes, mx6_tile.h).
+LSK_DEV void store_planes(uint8_t* dst, const int (&q)[32]) {
+  uint32_t hi[6] = {0, 0, 0, 0, 0, 0}, lo[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < 32; ++i) {
+    const uint32_t m = (uint32_t)(q[i] < 0 ? -q[i] : q[i]), sg = ((uint32_t)q[i] >> 31) << 5;
+    const uint32_t h = sg | (m >> 4), l = sg | (m & 15u);
+    const int bit = 6 * i, w = bit >> 5, o = bit & 31;
+    hi[w] |= h << o;
+    lo[w] |= l << o;
+    if (o > 26) {
+      hi[w + 1] |= h >> (32 - o);
+      lo[w + 1] |= l >> (32 - o);
+    }
+  }
+  // (each group of two words apart from its neighbours too, see store16_split)
+  store16_split(dst, hi[0], hi[1], hi[2], hi[3]);
+  __asm__ volatile("" ::: "memory");
+  store16_split(dst + 16, hi[4], hi[5], lo[4], lo[5]);
+  __asm__ volatile("" ::: "memory");
+  store16_split(dst + 32, lo[0], lo[1], lo[2], lo[3]);
+}
+
+// The block of 32 bf16 values at src (16-byte aligned) quantised by s (r = fl32(1 / s)).
+LSK_DEV void quant_block(const uint16_t* src, float s, float r, uint8_t* dst) {
+  int q[32];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const uint4 u = *(const uint4*)(src + 8 * c);
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      q[8 * c + 2 * j] = (int)fminf(fmaxf(rint_div8(bf16_to_f32((uint16_t)(w[j] & 0xffff)), s, r), -127.0f), 127.0f);
+      q[8 * c + 2 * j + 1] = (int)fminf(fmaxf(rint_div8(bf16_to_f32((uint16_t)(w[j] >> 16)), s, r), -127.0f), 127.0f);
+    }
+  }
+  store_planes(dst, q);
+}
+
+// The row quant of x [T, H] bf16 (16-byte aligned rows, H % 32 == 0) as six-bit planes [T, H / 32 * 48
+// bytes]: one block of 128 threads per row, a thread per 32-wide block in the second pass (the row
+// is in the L1 then).
+__global__ __launch_bounds__(128) void rowquant_mx6_kernel(const uint16_t* __restrict__ x, int64_t H,
+                                                           uint8_t* __restrict__ q, float* __restrict__ asc) {
+  __shared__ float red[2];
+  const int64_t t = blockIdx.x;
+  const uint16_t* row = x + t * H;
+  const int c8 = (int)(H / 8), nb = (int)(H / 32);
+  float am = 0.0f;
+  for (int i = threadIdx.x; i < c8; i += 128) {
+    float v[8];
+    load8_as_f32<LSK_BF16>(row, i, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(v[e]));
+  }
+  am = block_max<128>(am, red);
+  const float s = f32_div(fmaxf(am, kAmaxFloor), 127.0f), rs = f32_div(1.0f, s);
+  if (threadIdx.x == 0) asc[t] = s;
+  for (int b = threadIdx.x; b < nb; b += 128) quant_block(row + 32 * b, s, rs, q + (t * nb + b) * 48);
+}
+
+// requant_bf16_kernel's rows as six-bit planes, a thread per 32-wide block.
+__global__ __launch_bounds__(256) void requant_mx6_kernel(const uint16_t* __restrict__ h, const uint32_t* __restrict__ amax,
+                                                          const int32_t* __restrict__ nrows, int I,
+                                                          uint8_t* __restrict__ q, float* __restrict__ asc) {
+  const int nb = I / 32;
+  const int64_t total = (int64_t)*nrows * nb;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+    const int64_t p = i / nb;
+    const int b = (int)(i - p * nb);
+    const float s = f32_div(fmaxf(__uint_as_float(amax[p]), kAmaxFloor), 127.0f), rs = f32_div(1.0f, s);
+    if (b == 0) asc[p] = s;
+    quant_block(h + p * I + 32 * b, s, rs, q + i * 48);
   }
 }
 
@@ -475,6 +552,216 @@ __global__ __launch_bounds__(256, RING == 2 ? 3 : 2) void moe_mx_pp_kernel(lsk::
   moe_mx_epilogue<MODE>(a, acc, nt, p0, p1, bias, mx_smem);
 }
 
+// The activation table's entries of gate values 2^-9 <= |g| < 2^11, copied to LDS for a tile's
+// epilogue (20 KB, each sign's run contiguous): gathered from memory, every lookup is a cache line
+// of its own, which was a quarter of the gate/up launch (GPT-OSS-20B at 4096 tokens, 240 us).
+// Values outside are read from memory.
+constexpr int kActE0 = 118, kActRun = 20 * 128;
+
+// Whether no output of a row with scale asc, routing weight w and column bias b can be NaN, given
+// the accumulators' bound of 2^81 (E8M0 bytes up to kMx6QuietKexp and K < 2^18: 2^13 blocks of 2^15
+// 2^53): finite scales and biases keep every product and sum finite.
+constexpr int kMx6QuietKexp = 180;
+
+// Two binary32 values rounded to bf16, packed; QUIET: neither is NaN.
+template <bool QUIET>
+LSK_DEV uint32_t pack2(float a, float b) {
+  return QUIET ? pack_bf16x2_nonan(a, b) : pack_bf16x2(a, b);
+}
+LSK_DEV float lo_f32(uint32_t p) { return __uint_as_float(p << 16); }
+LSK_DEV float hi_f32(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
+
+// The epilogue of a six-bit tile.  Each wave stages a strip of 32 rows through its part of the drained
+// ring and walks it in a loop that is not unrolled: the code runs once per tile, so every 64 bytes of
+// it cost an instruction-cache miss (unrolled over the accumulators it was 60 KB, and 250 of the
+// gate/up launch's 830 us at GPT-OSS-20B with 4096 tokens).  A lane takes four columns: MODE 0 of 32
+// h columns, gate values first and up values 32 columns on; MODE 1 of 64.  s_asc / s_w / s_off: the
+// tile rows' scales, routing weights and byte offsets in the output (beyond its resource for absent
+// rows).
+constexpr int kMx6Ldc = 68;
+template <int MODE, bool QUIET>
+LSK_DEV void mx6_epilogue(const lsk::MoeGemmArgs& a, const lsk::Mx6Cfg::Acc& acc, int na, int p0, int p1, int nt, int wm,
+                          int wn, const float* bias, __amdgpu_buffer_rsrc_t ro, const float* s_asc, const float* s_w,
+                          const uint32_t* s_off, float* region, const float* s_tab) {
+  using C = lsk::Mx6Cfg;
+  const int lane = threadIdx.x & 63;
+  constexpr int kLanes = MODE == 0 ? 8 : 16, kRows = 64 / kLanes;  // lanes per row, rows per pass
+  const int c4 = lane % kLanes * 4, r0 = lane / kLanes;
+  const int col = MODE == 0 ? nt * 64 + wn * 32 + c4 : nt * 128 + wn * 64 + c4;
+  const bool cok = col < a.N;  // (N % 32 == 0: whole quads)
+  float b0[4], b1[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    b0[t] = bias && cok ? bias[col + t] : 0.0f;
+    b1[t] = MODE == 0 && bias && cok ? bias[a.N + col + t] : 0.0f;
+  }
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i) {
+    if (i >= na) break;
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        region[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * kMx6Ldc + j * 32 + (lane & 31)] = acc[i][j][r];
+#pragma unroll 1
+    for (int row = r0; row < 32; row += kRows) {
+      const int tr = wm * 64 + i * 32 + row;
+      const float asc = s_asc[tr];
+      const uint32_t off = s_off[tr];
+      // bfr(acc * asc), then bfr(+ bias)
+      auto quad = [&](const float* src, const float (&b)[4], float (&y)[4]) {
+        const v4f v = *(const v4f*)src;
+#pragma unroll
+        for (int t = 0; t < 4; t += 2) {
+          uint32_t p = pack2<QUIET>(f32_mul(v[t], asc), f32_mul(v[t + 1], asc));
+          if (bias) p = pack2<QUIET>(f32_add(lo_f32(p), b[t]), f32_add(hi_f32(p), b[t + 1]));
+          y[t] = lo_f32(p);
+          y[t + 1] = hi_f32(p);
+        }
+      };
+      float y[4];
+      quad(region + row * kMx6Ldc + c4, b0, y);
+      if constexpr (MODE == 0) {
+        float u[4];
+        quad(region + row * kMx6Ldc + 32 + c4, b1, u);
+        float am = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const uint32_t bits = __float_as_uint(y[t]) >> 16;
+          const uint32_t k = (bits & 0x7fffu) - kActE0 * 128;
+          const bool in = k < (uint32_t)kActRun;
+          float e = s_tab[in ? (bits >> 15) * kActRun + k : 0];
+          if (!in) e = a.act_tab[bits];
+          y[t] = lsk::act_from_entry(a.act, e, u[t]);
+          am = fmaxf(am, fabsf(y[t]));
+        }
+        // the row's maximum over its eight lanes
+        uint32_t m = cok ? __float_as_uint(am) : 0u;
+        m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xb1, 0xf, 0xf, false));
+        m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4e, 0xf, 0xf, false));
+        m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, false));
+        if (c4 == 0 && p0 + tr < p1) atomicMax(&a.h_amax[p0 + tr], m);
+      } else {
+        const float w = s_w[tr];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) y[t] = f32_mul(w, y[t]);
+      }
+      if (cok)
+        __builtin_amdgcn_raw_buffer_store_b64(v2u32{pack2<QUIET>(y[0], y[1]), pack2<QUIET>(y[2], y[3])}, ro,
+                                              off + 2 * col, 0, 0);
+    }
+  }
+}
+
+// Six-bit tiles on the block-scaled MFMA (mx6_tile.h), per-row activation scales.  MODE 0: a wave's
+// first 32 columns are gate rows and its second the up rows of the same h columns, so a lane holds
+// both values of an output; MODE 1: 128 weight rows in order.
+template <int MODE>
+__global__ __launch_bounds__(256, 2) void moe_mx6_kernel(lsk::MoeGemmArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char mx_smem[];
+  using C = lsk::Mx6Cfg;
+  const int ntiles = MODE == 0 ? (a.N + 63) / 64 : (a.N + 127) / 128;
+  const int L = lsk::xcd_logical_id(blockIdx.x, gridDim.x);
+  const int mt = L / ntiles, nt = L - mt * ntiles;
+  if (mt >= a.tiles[0]) return;
+  const int e = a.tiles[1 + 2 * mt];
+  const int p0 = a.tiles[2 + 2 * mt];
+  const int p1 = min(a.offs[e + 1], p0 + lsk::kMoeBM);
+  const float* bias = a.b_ptrs ? (const float*)wave_uniform64(a.b_ptrs[e]) : nullptr;
+  const int nrows_w = MODE == 0 ? 2 * a.N : a.N;
+  const __amdgpu_buffer_rsrc_t ra = lsk::make_rsrc(a.A, a.a_bytes);
+  const __amdgpu_buffer_rsrc_t rb = lsk::make_rsrc((const void*)wave_uniform64(a.w_ptrs[e]), a.w_bytes);
+  const __amdgpu_buffer_rsrc_t rs =
+      lsk::make_rsrc((const void*)wave_uniform64(a.ws_ptrs[e]), (int64_t)nrows_w * a.lds);
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+  // the wave's quarter: the row halves swap SIMDs from tile to tile, as the upper half of a tile is
+  // often empty
+  const int wn = wave & 1, wm = (wave >> 1) ^ (L & 1);
+  const int left = p1 - p0 - wm * 64;
+  const int na = left <= 0 ? 0 : (left <= 32 ? 1 : 2);
+  auto wrow = [&](int r) -> int {
+    if (MODE == 0) {
+      const int hc = nt * 64 + (r >> 6) * 32 + (r & 31);
+      return hc < a.N ? ((r >> 5) & 1 ? a.N + hc : hc) : -1;
+    }
+    const int n = nt * 128 + r;
+    return n < a.N ? n : -1;
+  };
+  // the epilogue's operands of tile row tid, requested before the loop
+  float o_asc = 0.0f, o_w = 1.0f;
+  uint32_t o_off = lsk::kOob;
+  if (tid < C::BM && p0 + tid < p1) {
+    const int p = p0 + tid;
+    o_asc = a.a_scale[MODE == 0 ? a.row_tok[p] : p];
+    if (MODE == 1 && a.row_w) o_w = a.row_w[p];
+    o_off = MODE == 0 ? (uint32_t)(tid * a.N * 2) : (uint32_t)((a.row_dst ? a.row_dst[p] : p) * a.N * 2);
+  }
+  const lsk::Mx6Rows rows = lsk::mx6_rows(
+      [&](int r) -> uint32_t {
+        const int p = p0 + r;
+        if (p >= p1) return lsk::kOob;
+        return (uint32_t)((int64_t)(MODE == 0 ? a.row_tok[p] : p) * a.lda);
+      },
+      [&](int r) -> uint32_t {
+        const int w = wrow(r);
+        return w >= 0 ? (uint32_t)((int64_t)w * a.ldw) : lsk::kOob;
+      },
+      [&](int r) -> uint32_t {
+        const int w = wrow(r);
+        return w >= 0 ? (uint32_t)((int64_t)w * a.lds) : lsk::kOob;
+      });
+  C::Acc acc;
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+  if (na == 2) lsk::mx6_mainloop<2>(acc, ra, rb, rs, rows, a.K, wm, wn, mx_smem);
+  else if (na == 1) lsk::mx6_mainloop<1>(acc, ra, rb, rs, rows, a.K, wm, wn, mx_smem);
+  else lsk::mx6_mainloop<0>(acc, ra, rb, rs, rows, a.K, wm, wn, mx_smem);
+
+  float* s_asc = (float*)(mx_smem + C::kRowOff);
+  float* s_w = s_asc + C::BM;
+  uint32_t* s_off = (uint32_t*)(s_w + C::BM);
+  // over the drained ring: the waves' strips, then the table's run
+  constexpr int kStrip = 32 * kMx6Ldc * 4, kTabOff = 4 * kStrip;
+  static_assert(kTabOff + 8 * kActRun <= C::kRowOff, "the epilogue's LDS lies inside the ring");
+  float* region = (float*)(mx_smem + wave * kStrip);
+  const float* s_tab = (const float*)(mx_smem + kTabOff);
+  __syncthreads();  // every wave is past its last read of it
+  if constexpr (MODE == 0) {
+    const __amdgpu_buffer_rsrc_t rt = lsk::make_rsrc(a.act_tab, 65536 * 4);
+#pragma unroll
+    for (int j = 0; j < 2 * kActRun / 1024; ++j) {
+      const int p = j * 256 + tid;  // 16-byte chunk
+      const int sign = p >= kActRun / 4;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rt, (lsk::lds_void_t)(mx_smem + kTabOff + (j * 256 + wave * 64) * 16), 16,
+          (sign * 32768 + kActE0 * 128 + (p - sign * (kActRun / 4)) * 4) * 4, 0, 0, 0);
+    }
+  }
+  if (tid < C::BM) {
+    s_asc[tid] = o_asc;
+    s_w[tid] = o_w;
+    s_off[tid] = o_off;
+  }
+  lsk::compiler_fence();
+  lsk::wait_vm<0>();
+  const int quiet = __syncthreads_and(!(tid < C::BM) || (fabsf(o_asc) < 0x1p40f && fabsf(o_w) < 0x1p40f));
+  if (na == 0) return;
+  const __amdgpu_buffer_rsrc_t ro = MODE == 0 ? lsk::make_rsrc(a.h + (int64_t)p0 * a.N, (int64_t)(p1 - p0) * a.N * 2)
+                                              : lsk::make_rsrc(a.y, a.y_bytes);
+  bool qb = a.mx6 == 2 && quiet;
+  if (bias) {
+    const int col = MODE == 0 ? nt * 64 + wn * 32 + (lane & 31) : nt * 128 + wn * 64 + lane;
+    const bool ok = col >= a.N || (fabsf(bias[col]) < 0x1p96f && (MODE == 1 || fabsf(bias[a.N + col]) < 0x1p96f));
+    qb = qb && __builtin_amdgcn_ballot_w64(!ok) == 0;
+  }
+  if (qb) mx6_epilogue<MODE, true>(a, acc, na, p0, p1, nt, wm, wn, bias, ro, s_asc, s_w, s_off, region, s_tab);
+  else mx6_epilogue<MODE, false>(a, acc, na, p0, p1, nt, wm, wn, bias, ro, s_asc, s_w, s_off, region, s_tab);
+}
+
 // ---------------------------------------------------------------- dequant and packing
 __global__ __launch_bounds__(256) void dequant_mxfp4_kernel(const uint8_t* __restrict__ packed,
                                                             const uint8_t* __restrict__ scale, int64_t rows, int64_t K,
@@ -544,6 +831,16 @@ int launch_grouped(const lsk::MoeGemmArgs& ga, int64_t max_tiles, hipStream_t s)
   const int64_t blocks = max_tiles * ntiles;
   if (blocks == 0) return LSK_OK;
   LSK_REQUIRE(blocks <= 0x7fffffff, "moe_mx_gemm_kernel: grid too large");
+  if (ga.mx6) {
+    static std::atomic<bool> attr_6{false};
+    auto kern = moe_mx6_kernel<MODE>;
+    if (!attr_6) {
+      if (int rc = reserve_lds(kern, lsk::Mx6Cfg::kSmemBytes, "moe_mx6_kernel")) return rc;
+      attr_6 = true;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), lsk::Mx6Cfg::kSmemBytes, s, ga);
+    return lsk::check_launch(MODE == 0 ? "moe_mx6_kernel<gate_up>" : "moe_mx6_kernel<down>");
+  }
   if (ga.mx2 >= 2) {
     static std::atomic<bool> attr_rs{false};
     auto kern = moe_mx_gemm_kernel<MODE, true, true>;
@@ -1287,6 +1584,19 @@ int launch_blockquant_mx2(const uint16_t* x, int64_t ldx, int64_t R, const int32
   hipLaunchKernelGGL(blockquant_mx2_kernel, dim3((unsigned)R), dim3(256), 0, s, x, ldx, nrows, K, q, ka, flag, any, lo,
                      hi);
   return check_launch("blockquant_mx2_kernel");
+}
+
+int launch_rowquant_mx6(const uint16_t* x, int64_t T, int64_t H, uint8_t* q, float* asc, hipStream_t s) {
+  if (T == 0) return LSK_OK;
+  LSK_REQUIRE(T <= 0x7fffffff, "rowquant_mx6: too many rows");
+  hipLaunchKernelGGL(rowquant_mx6_kernel, dim3((unsigned)T), dim3(128), 0, s, x, H, q, asc);
+  return check_launch("rowquant_mx6_kernel");
+}
+
+int launch_requant_mx6(const uint16_t* h, const uint32_t* amax, const int32_t* nrows, int64_t R, int I, uint8_t* q,
+                       float* asc, hipStream_t s) {
+  hipLaunchKernelGGL(requant_mx6_kernel, dim3(grid_for(R * (I / 32))), dim3(256), 0, s, h, amax, nrows, I, q, asc);
+  return check_launch("requant_mx6_kernel");
 }
 
 int launch_requant_bf16(const uint16_t* h, const uint32_t* amax, const int32_t* nrows, int64_t R, int I, uint16_t* q,

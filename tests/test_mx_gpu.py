@@ -407,3 +407,44 @@ def test_moe_mx_grouped_main_loops(mxv, big_exp):
     with np.errstate(over="ignore", invalid="ignore"):
         ref = C.moe_forward_mx(x, oexp, idx, w, C.act_swigluoai)
     assert np.array_equal(u16(y), ref)
+
+
+@pytest.mark.parametrize("act", ["silu", "swigluoai"])
+@pytest.mark.parametrize("T,E,k,H,I,bias,big", [(257, 4, 2, 96, 160, False, False), (600, 3, 2, 352, 224, True, False),
+                                                (300, 40, 1, 64, 32, True, False), (513, 5, 3, 288, 96, False, True),
+                                                (1200, 2, 1, 32, 128, True, True)])
+def test_moe_mx_six_bit_tiles(act, T, E, k, H, I, bias, big):
+    """Layers past 256 tokens on the block-scaled MFMA tiles against the oracle: one to eleven MX
+    blocks (K stages of four), experts of no rows up to several 128-row tiles, empty and partial
+    32-row strips, partial column tiles, every int8 magnitude (a row of extreme values), gate values
+    inside and outside the table's run in LDS, and with `big` the outermost exponent bytes these
+    tiles take (16 and 239, which also turn the NaN-free epilogue off)."""
+    from lockstep_amd import moe_ref as MR
+    from lockstep_amd import workloads as WL
+    say("mx six-bit tiles", act, T, E, k, H, I, bias, big)
+    x, experts, logits = WL.moe_mx_inputs(T, E, k, H, I, seed=T + H, bias=bias)
+    x[3] = 0.0
+    x[5] = C.bfr((np.arange(H, dtype=F32) - H // 2) * F32(1e-3))
+    x[7] *= F32(2.0 ** -14)
+    if big:
+        for j, (p13, s13, p2, s2, b13, b2) in enumerate(experts):
+            s13, s2 = s13.copy(), s2.copy()
+            s13[::5, 0] = 16
+            s2[::7, 1] = 239
+            s2[1::7, 0] = 16
+            experts[j] = (p13, s13, p2, s2, b13, b2)
+    idx, w = routing_from_logits(logits, k)
+    oexp, dexp = [], []
+    for (p13, s13, p2, s2, b13, b2) in experts:
+        m13, _ = C.mx_to_m2(p13, s13)
+        m2_, _ = C.mx_to_m2(p2, s2)
+        oexp.append(((m13, s13), (m2_, s2), b13, b2))
+        dexp.append(((to_dev(p13), to_dev(s13)), (to_dev(p2), to_dev(s2)), None if b13 is None else to_dev(b13),
+                     None if b2 is None else to_dev(b2)))
+    tables = MR.ExpertTablesMX(dexp, packed=True)
+    ridx, rw = routing_device(idx, w)
+    y, _, _ = MR.moe_forward_mx(bf16_dev(x), None, tables, k, True, _tab(), 0, getattr(MR, "act_" + act),
+                                routing=(ridx, rw))
+    with np.errstate(over="ignore", invalid="ignore"):
+        ref = C.moe_forward_mx(x, oexp, idx, w, getattr(C, "act_" + act))
+    assert np.array_equal(u16(y), ref), int((u16(y) != ref).sum())
