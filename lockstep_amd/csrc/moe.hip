@@ -15,6 +15,7 @@
 //   6. combine: per token, binary32 adds of its slots in ascending expert order from +0.
 #include <atomic>
 
+#include "act_run.h"
 #include "contract_act.h"
 #include "mfma_tile.h"
 #include "moe_internal.h"
@@ -833,31 +834,40 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, char* smem_moe, M
     sc_ws[tid] = c_ws;
     sc_b[tid] = c_b;
   }
+  // the activation table's common range behind the staged rows (half a strip a wave; the skinny path's
+  // whole strips of one row of waves)
+  constexpr int kStaged = (C::kThreads / 64) * (C::kStripBytes / 2);
+  constexpr int kTabOff = kStaged > C::kWN * C::kStripBytes ? kStaged : C::kWN * C::kStripBytes;
+  static_assert(kTabOff + lsk::kActRunBytes <= C::kScaleOff, "the epilogue's LDS lies below the operands");
+  const float* s_tab = (const float*)(smem_moe + kTabOff);
+  if (MODE == 0 && a.act_tab) {
+    lsk::act_run_load(a.act_tab, smem_moe + kTabOff, wave, C::kThreads / 64);
+    lsk::compiler_fence();
+    lsk::wait_vm<0>();
+  }
   __syncthreads();
 
-  int32_t* region = (int32_t*)(smem_moe + wave * C::kStripBytes);
-  auto strip = [&](int i) {
-    if (MODE == 0) {
-      // a wave strip is 32 rows x P [gate 32 | up 32] pairs; 8 lanes cover a pair's 32 columns
-      // by quads, LPR lanes a row.  First every pass's gate / up values (and, with the table, all
-      // their table entries, gathered together so that one latency covers the strip), then the
-      // activations, the stores and the row maxima.
-      constexpr int P = C::WTN / 64, LPR = 8 * P, RPP = 64 / LPR, NP = 32 / RPP;
+  // The rows of a staged region (its row 0 is tile row m0), in a loop that is not unrolled: the code
+  // runs once per tile, so every 64 bytes of it cost an instruction-cache miss.
+  auto rows = [&](const int32_t* region, int m0, int n) {
+    if constexpr (MODE == 0) {
+      // rows of P [gate 32 | up 32] pairs; 8 lanes cover a pair's 32 columns by quads, LPR lanes a row
+      constexpr int P = C::WTN / 64, LPR = 8 * P, RPP = 64 / LPR;
       const int pr = (lane >> 3) % P;
       const int c4 = (lane & 7) * 4;
       const int hc0 = nt * 128 + wn * (32 * P) + pr * 32 + c4;
+      const bool whole = hc0 + 4 <= a.N;
       // this lane's four gate and four up columns: the same in every pass
       const int cg0 = wn * C::WTN + pr * 64 + c4;
       const v4f wsg = *(const v4f*)(sc_ws + cg0), wsu = *(const v4f*)(sc_ws + cg0 + 32);
       const v4f bg = *(const v4f*)(sc_b + cg0), bu = *(const v4f*)(sc_b + cg0 + 32);
-      float gv[NP][4], uv[NP][4];
-#pragma unroll
-      for (int t = 0; t < NP; ++t) {
-        const int row = lane / LPR + RPP * t;
-        const int ml = wm * C::WTM + i * 32 + row;
+#pragma unroll 1
+      for (int row = lane / LPR; row < n; row += RPP) {
+        const int p = p0 + m0 + row;
         const v4i vg = *(const v4i*)(region + row * C::kLdc + pr * 64 + c4);
         const v4i vu = *(const v4i*)(region + row * C::kLdc + pr * 64 + 32 + c4);
-        const float asc = sc_asc[ml];  // 0 past the tile's rows
+        const float asc = sc_asc[m0 + row];  // 0 past the tile's rows
+        float hv[4], am = 0.0f;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           float yg = bfr(f32_mul(f32_mul((float)vg[q], wsg[q]), asc));
@@ -866,116 +876,73 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, char* smem_moe, M
             yg = bfr(f32_add(yg, bg[q]));
             yu = bfr(f32_add(yu, bu[q]));
           }
-          gv[t][q] = yg;
-          uv[t][q] = yu;
+          hv[q] = a.act_tab ? lsk::act_from_entry(a.act, lsk::act_run_entry(s_tab, a.act_tab, yg), yu)
+                            : lsk::act_eval(a.act, yg, yu, a.frac, nullptr);
+          if (whole || hc0 + q < a.N) am = fmaxf(am, fabsf(hv[q]));
         }
-      }
-      if (a.act_tab) {
-#pragma unroll
-        for (int t = 0; t < NP; ++t)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) gv[t][q] = a.act_tab[__float_as_uint(gv[t][q]) >> 16];
-      }
-#pragma unroll
-      for (int t = 0; t < NP; ++t) {
-        const int row = lane / LPR + RPP * t;
-        const int ml = wm * C::WTM + i * 32 + row;
-        const int p = p0 + ml;
-        float am = 0.0f;
-        if (p < p1 && hc0 + 4 <= a.N) {
-          // a whole quad: no column tests
-          float hv[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            hv[q] = a.act_tab ? lsk::act_from_entry(a.act, gv[t][q], uv[t][q])
-                              : lsk::act_eval(a.act, gv[t][q], uv[t][q], a.frac, nullptr);
-            am = fmaxf(am, fabsf(hv[q]));
-          }
-          *(uint2*)(a.h + (int64_t)p * a.N + hc0) = make_uint2(pack_bf16x2(hv[0], hv[1]), pack_bf16x2(hv[2], hv[3]));
-        } else if (p < p1) {
-          uint16_t hb[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            hb[q] = 0;
-            if (hc0 + q < a.N) {
-              const float hv = a.act_tab ? lsk::act_from_entry(a.act, gv[t][q], uv[t][q])
-                                         : lsk::act_eval(a.act, gv[t][q], uv[t][q], a.frac, nullptr);
-              hb[q] = f32_to_bf16(hv);
-              am = fmaxf(am, fabsf(hv));
-            }
-          }
+        if (p < p1) {
           uint16_t* dst = a.h + (int64_t)p * a.N + hc0;
-          if (hc0 + 4 <= a.N) {
-            *(uint2*)dst =
-                make_uint2((uint32_t)hb[0] | ((uint32_t)hb[1] << 16), (uint32_t)hb[2] | ((uint32_t)hb[3] << 16));
+          if (whole) {
+            *(uint2*)dst = make_uint2(pack_bf16x2(hv[0], hv[1]), pack_bf16x2(hv[2], hv[3]));
           } else {
+#pragma unroll
             for (int q = 0; q < 4; ++q)
-              if (hc0 + q < a.N) dst[q] = hb[q];
+              if (hc0 + q < a.N) dst[q] = f32_to_bf16(hv[q]);
           }
         }
-#pragma unroll
-        for (int o = 1; o < LPR; o <<= 1) am = fmaxf(am, __shfl_xor(am, o, 64));
-        if (lane % LPR == 0 && p < p1) atomicMax(&a.h_amax[p], __float_as_uint(am));
+        uint32_t m = __float_as_uint(am);
+        m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xb1, 0xf, 0xf, false));
+        m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4e, 0xf, 0xf, false));
+        m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, false));
+        if (LPR == 16) m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x140, 0xf, 0xf, false));
+        if (lane % LPR == 0 && p < p1) atomicMax(&a.h_amax[p], m);
       }
     } else {
-      // 32 rows x QPR column quads; a lane keeps one quad
+      // QPR column quads a row; a lane keeps one quad
       constexpr int QPR = C::WTN / 4, RPP = 64 / QPR;
       const int c4 = (lane % QPR) * 4;
-      const int n0 = nt * 256 + wn * C::WTN + c4;
-      // this lane's four columns: the same in every pass
       const int cl0 = wn * C::WTN + c4;
+      const int n0 = nt * 256 + cl0;
+      const bool whole = n0 + 4 <= a.N;
       const v4f wsq = *(const v4f*)(sc_ws + cl0), bq = *(const v4f*)(sc_b + cl0);
-#pragma unroll
-      for (int t = 0; t < 32 / RPP; ++t) {
-        const int row = lane / QPR + RPP * t;
-        const int ml = wm * C::WTM + i * 32 + row;
-        const int p = p0 + ml;
+#pragma unroll 1
+      for (int row = lane / QPR; row < n; row += RPP) {
+        const int ml = m0 + row;
+        if (p0 + ml >= p1 || n0 >= a.N) continue;
         const v4i v = *(const v4i*)(region + row * C::kLdc + c4);
-        if (p < p1 && n0 + 4 <= a.N) {
-          // a whole quad: no column tests
-          const float asc = sc_asc[ml];
-          const float wt = sc_w[ml];
-          float o[4];
+        const float asc = sc_asc[ml], wt = sc_w[ml];
+        float o[4];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            float yv = bfr(f32_mul(f32_mul((float)v[q], wsq[q]), asc));
-            if (bias) yv = bfr(f32_add(yv, bq[q]));
-            o[q] = f32_mul(wt, yv);
-          }
-          *(uint2*)(a.y + (int64_t)sc_dst[ml] * a.N + n0) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-        } else if (p < p1 && n0 < a.N) {
-          const float asc = sc_asc[ml];
-          const float wt = sc_w[ml];
-          uint16_t ob[4];
+        for (int q = 0; q < 4; ++q) {
+          float yv = bfr(f32_mul(f32_mul((float)v[q], wsq[q]), asc));
+          if (bias) yv = bfr(f32_add(yv, bq[q]));
+          o[q] = f32_mul(wt, yv);
+        }
+        uint16_t* dst = a.y + (int64_t)sc_dst[ml] * a.N + n0;
+        if (whole) {
+          *(uint2*)dst = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+        } else {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int cl = wn * C::WTN + c4 + q;
-            ob[q] = 0;
-            if (n0 + q < a.N) {
-              float yv = bfr(f32_mul(f32_mul((float)v[q], sc_ws[cl]), asc));
-              if (bias) yv = bfr(f32_add(yv, sc_b[cl]));
-              ob[q] = f32_to_bf16(f32_mul(wt, yv));
-            }
-          }
-          uint16_t* dst = a.y + (int64_t)sc_dst[ml] * a.N + n0;
-          if (n0 + 4 <= a.N) {
-            *(uint2*)dst =
-                make_uint2((uint32_t)ob[0] | ((uint32_t)ob[1] << 16), (uint32_t)ob[2] | ((uint32_t)ob[3] << 16));
-          } else {
-            for (int q = 0; q < 4; ++q)
-              if (n0 + q < a.N) dst[q] = ob[q];
-          }
+          for (int q = 0; q < 4; ++q)
+            if (n0 + q < a.N) dst[q] = f32_to_bf16(o[q]);
         }
       }
     }
   };
-  if (na > 0) {
-    if (!skinny) lsk::pp_stage_strip<C::TN, C::kLdc>(acc[0], region);
-    strip(0);
+  if (skinny) {  // the sums of up to 32 rows, in the first row of waves' regions
+    if (na > 0) rows((const int32_t*)(smem_moe + wave * C::kStripBytes), 0, 32);
+    return;
   }
-  if (na > 1) {
-    lsk::pp_stage_strip<C::TN, C::kLdc>(acc[1], region);
-    strip(1);
+  // 16 rows at a time through the wave's own region
+  int32_t* region = (int32_t*)(smem_moe + wave * (C::kStripBytes / 2));
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i) {
+    if (i >= na) break;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      lsk::stage_half<C::TN, C::kLdc>(acc[i], h, region);
+      rows(region, wm * C::WTM + i * 32 + h * 16, 16);
+    }
   }
 }
 
@@ -2889,7 +2856,9 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
   g1.N = (int)I;
   g1.act = a->act;
   g1.frac = a->frac;
-  g1.act_tab = a->act_tab;
+  // (the ping-pong tiles copy 16-byte pieces of the table; without it they evaluate the activation, the
+  // same bits)
+  g1.act_tab = use_pp && !mx && ((uintptr_t)a->act_tab & 15) ? nullptr : a->act_tab;
   g1.h = w.h;
   g1.h_amax = w.h_amax;
   g1.lds = a->lds13;

@@ -2,6 +2,7 @@
 // E2M1/E8M0 dequant, and the doubled-mantissa packer.  See mx_tile.h for the exactness argument.
 #include <atomic>
 
+#include "act_run.h"
 #include "contract_act.h"
 #include "moe_internal.h"
 #include "moe_route.h"
@@ -552,12 +553,6 @@ __global__ __launch_bounds__(256, RING == 2 ? 3 : 2) void moe_mx_pp_kernel(lsk::
   moe_mx_epilogue<MODE>(a, acc, nt, p0, p1, bias, mx_smem);
 }
 
-// The activation table's entries of gate values 2^-9 <= |g| < 2^11, copied to LDS for a tile's
-// epilogue (20 KB, each sign's run contiguous): gathered from memory, every lookup is a cache line
-// of its own, which was a quarter of the gate/up launch (GPT-OSS-20B at 4096 tokens, 240 us).
-// Values outside are read from memory.
-constexpr int kActE0 = 118, kActRun = 20 * 128;
-
 // Whether no output of a row with scale asc, routing weight w and column bias b can be NaN, given
 // the accumulators' bound of 2^81 (E8M0 bytes up to kMx6QuietKexp and K < 2^18: 2^13 blocks of 2^15
 // 2^53): finite scales and biases keep every product and sum finite.
@@ -627,12 +622,7 @@ LSK_DEV void mx6_epilogue(const lsk::MoeGemmArgs& a, const lsk::Mx6Cfg::Acc& acc
         float am = 0.0f;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const uint32_t bits = __float_as_uint(y[t]) >> 16;
-          const uint32_t k = (bits & 0x7fffu) - kActE0 * 128;
-          const bool in = k < (uint32_t)kActRun;
-          float e = s_tab[in ? (bits >> 15) * kActRun + k : 0];
-          if (!in) e = a.act_tab[bits];
-          y[t] = lsk::act_from_entry(a.act, e, u[t]);
+          y[t] = lsk::act_from_entry(a.act, lsk::act_run_entry(s_tab, a.act_tab, y[t]), u[t]);
           am = fmaxf(am, fabsf(y[t]));
         }
         // the row's maximum over its eight lanes
@@ -726,20 +716,12 @@ __global__ __launch_bounds__(256, 2) void moe_mx6_kernel(lsk::MoeGemmArgs a) {
   uint32_t* s_off = (uint32_t*)(s_w + C::BM);
   // over the drained ring: the waves' strips, then the table's run
   constexpr int kStrip = 32 * kMx6Ldc * 4, kTabOff = 4 * kStrip;
-  static_assert(kTabOff + 8 * kActRun <= C::kRowOff, "the epilogue's LDS lies inside the ring");
+  static_assert(kTabOff + lsk::kActRunBytes <= C::kRowOff, "the epilogue's LDS lies inside the ring");
   float* region = (float*)(mx_smem + wave * kStrip);
   const float* s_tab = (const float*)(mx_smem + kTabOff);
   __syncthreads();  // every wave is past its last read of it
   if constexpr (MODE == 0) {
-    const __amdgpu_buffer_rsrc_t rt = lsk::make_rsrc(a.act_tab, 65536 * 4);
-#pragma unroll
-    for (int j = 0; j < 2 * kActRun / 1024; ++j) {
-      const int p = j * 256 + tid;  // 16-byte chunk
-      const int sign = p >= kActRun / 4;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rt, (lsk::lds_void_t)(mx_smem + kTabOff + (j * 256 + wave * 64) * 16), 16,
-          (sign * 32768 + kActE0 * 128 + (p - sign * (kActRun / 4)) * 4) * 4, 0, 0, 0);
-    }
+    lsk::act_run_load(a.act_tab, mx_smem + kTabOff, wave, 4);
   }
   if (tid < C::BM) {
     s_asc[tid] = o_asc;
