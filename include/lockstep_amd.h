@@ -420,8 +420,10 @@ typedef enum {
  *   top-k by s * E + (E - 1 - e) (ties to the lower index), in rank order;
  *   w = bf16(fl32(s_sel) / fl32(S)), S = sum of the selected (renormalize) or of all scores, >= 1.
  * g: [T, E] of g_dtype (LSK_F32 holding bf16 values, or LSK_BF16), row stride ldg;
- * tab: [8192] int32 (the FRAC table); idx: [T, k] int64; w_bf16: [T, k] bf16 bits.
+ * tab: [8192] int32 (the FRAC table), or with LSK_ROUTE_TAB64 added to renormalize (0 or 1) 8192 int64
+ * entries, of which the low 32 bits are read; idx: [T, k] int64; w_bf16: [T, k] bf16 bits.
  * E <= 1024, k <= min(E, 32). */
+#define LSK_ROUTE_TAB64 0x40000000
 int lsk_router_topk(const void* g, int g_dtype, int64_t ldg, int64_t T, int64_t E, int k, int renormalize,
                     const int32_t* tab, int64_t* idx, uint16_t* w_bf16, void* stream);
 

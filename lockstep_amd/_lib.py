@@ -18,6 +18,7 @@ LIB_PATH = os.path.join(HERE, "liblockstep_amd.so")
 LSK_F32, LSK_BF16, LSK_F16, LSK_I32, LSK_I8, LSK_BF16_AS_F32 = 0, 1, 2, 3, 4, 5
 EPI_V21, EPI_V2, EPI_POW2, EPI_RAW, EPI_V25 = 0, 1, 2, 3, 4
 LSK_ACT_SILU, LSK_ACT_SWIGLUOAI = 0, 1
+LSK_ROUTE_TAB64 = 0x40000000     # added to renormalize: the router table holds int64 entries
 
 _DTYPE = {torch.float32: LSK_F32, torch.bfloat16: LSK_BF16, torch.float16: LSK_F16,
           torch.int32: LSK_I32, torch.int8: LSK_I8}

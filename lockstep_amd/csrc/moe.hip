@@ -2305,13 +2305,14 @@ extern "C" int lsk_router_topk(const void* g, int g_dtype, int64_t ldg, int64_t 
   LSK_REQUIRE(T <= 0x7fffffffLL * 4, "lsk_router_topk: T too large");
   const dim3 grid((unsigned)((T + 3) / 4)), blk(256);
   hipStream_t s = (hipStream_t)stream;
+  const int rf = lsk::route_flags(renormalize);
   if (E <= 64) hipLaunchKernelGGL(router_topk_kernel<1>, grid, blk, 0, s, g, g_dtype, ldg, (int)T, (int)E, k,
-                                  renormalize, tab, idx, w_bf16);
+                                  rf, tab, idx, w_bf16);
   else if (E <= 128) hipLaunchKernelGGL(router_topk_kernel<2>, grid, blk, 0, s, g, g_dtype, ldg, (int)T, (int)E, k,
-                                        renormalize, tab, idx, w_bf16);
+                                        rf, tab, idx, w_bf16);
   else if (E <= 256) hipLaunchKernelGGL(router_topk_kernel<4>, grid, blk, 0, s, g, g_dtype, ldg, (int)T, (int)E, k,
-                                        renormalize, tab, idx, w_bf16);
-  else hipLaunchKernelGGL(router_topk_kernel<16>, grid, blk, 0, s, g, g_dtype, ldg, (int)T, (int)E, k, renormalize,
+                                        rf, tab, idx, w_bf16);
+  else hipLaunchKernelGGL(router_topk_kernel<16>, grid, blk, 0, s, g, g_dtype, ldg, (int)T, (int)E, k, rf,
                           tab, idx, w_bf16);
   return lsk::check_launch("router_topk_kernel");
 }
@@ -2647,6 +2648,7 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
   LSK_REQUIRE(a->x && a->w13_ptrs && a->ws13_ptrs && a->w2_ptrs && a->ws2_ptrs && a->frac && a->y,
               "lsk_moe_forward: null pointer");
   // the routing: given (idx, w), or computed here from the logits into (idx_out, w_out)
+  const int rflags = lsk::route_flags(a->renormalize);
   const int64_t* ridx = a->idx;
   const uint16_t* rwt = a->w;
   if (a->logits) {
@@ -2758,7 +2760,7 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
     const dim3 grid((unsigned)((T + 3) / 4)), blk(256);
 #define LSK_RRQ(EPLV, NXCV)                                                                                  \
   hipLaunchKernelGGL((moe_route_rowq_kernel<EPLV, NXCV>), grid, blk, 0, s, a->logits, a->logits_dtype,       \
-                     a->ld_logits, (int)T, (int)E, k, a->renormalize, a->router_tab, a->idx_out, a->w_out, a->x, \
+                     a->ld_logits, (int)T, (int)E, k, rflags, a->router_tab, a->idx_out, a->w_out, a->x, \
                      (int)H, w.qx, w.ascx)
 #define LSK_RRQ_E(NXCV) \
   if (E <= 64) LSK_RRQ(1, NXCV); else if (E <= 128) LSK_RRQ(2, NXCV); else LSK_RRQ(4, NXCV);
@@ -2817,7 +2819,7 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
     hipLaunchKernelGGL(moe_decode_prep_kernel, dim3((unsigned)(T + 1)), dim3(256), dsm, s, ridx, rwt, (int)T, k,
                        (int)E, w.offs, w.tiles, w.row_tok, w.row_dst, w.row_w, w.tok_cnt, w.h_amax, nzero,
                        a->x, (int)H, (void*)w.qx, w.ascx, mx ? 1 : 0, route_in_prep ? a->logits : nullptr,
-                       a->logits_dtype, a->ld_logits, a->router_tab, a->renormalize, a->idx_out, a->w_out, w.tiles2);
+                       a->logits_dtype, a->ld_logits, a->router_tab, rflags, a->idx_out, a->w_out, w.tiles2);
     if ((rc = lsk::check_launch("moe_decode_prep_kernel"))) return rc;
   } else if (nchunks == 1) {
     const size_t dsm = (size_t)(10 * E + 1) * 4 + (size_t)256 * k * 6;
@@ -2901,7 +2903,7 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
       ra.ldg = a->ld_logits;
       ra.E = (int)E;
       ra.k = k;
-      ra.renorm = a->renormalize;
+      ra.renorm = rflags;
       ra.rtab = a->router_tab;
       ra.x = a->x;
       ra.idx_out = a->idx_out;
@@ -2924,7 +2926,7 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
     const dim3 grid((unsigned)(k * nchunk));
 #define LSK_RG1(NCV, EPLV)                                                                                     \
   hipLaunchKernelGGL((moe_route_gemv1_kernel<NCV, 2, EPLV>), grid, dim3(256), 0, s, g1, w.gu, a->x, a->logits, \
-                     a->logits_dtype, (int)E, k, a->renormalize, a->router_tab, a->idx_out, a->w_out, w.offs,    \
+                     a->logits_dtype, (int)E, k, rflags, a->router_tab, a->idx_out, a->w_out, w.offs,             \
                      w.tiles, w.row_tok, w.row_dst, w.row_w, w.tok_cnt, w.ascx)
     const int nc = (int)((H + 1023) / 1024);
     if (E <= 128) {

@@ -7,6 +7,12 @@ namespace lsk {
 
 constexpr float kRouterC = 0x1.715476p+26f;  // fl32(2^26 / ln 2) (moe_ref.py:61)
 
+// The kernels' renorm flags from the C interface's renormalize (any value but the two with
+// LSK_ROUTE_TAB64 is a truth value).
+inline int route_flags(int renormalize) {
+  return (renormalize & ~1) == LSK_ROUTE_TAB64 ? 2 | (renormalize & 1) : (renormalize != 0 ? 1 : 0);
+}
+
 // One wave per token; lane l owns experts l, l + 64, ... (EPL per lane, E <= 64 * EPL).  The
 // reference's ranking key s * E + (E - 1 - e) orders like the pair (s, E - 1 - e); with scores
 // below 2^16 (entries of the FRAC table are at most 2^15, and a score is an entry shifted right) and
@@ -14,6 +20,9 @@ constexpr float kRouterC = 0x1.715476p+26f;  // fl32(2^26 / ln 2) (moe_ref.py:61
 // one DPP maximum over the wave and the winner is decoded from the wave-uniform key.  The
 // selection: lane r < k gets the rank-r expert e_r and its score s_r; S is the score sum the
 // weights divide by (the selected scores, or all of them without renormalisation), clamped to >= 1.
+// renorm: bit 0 renormalise, bit 1 the table's entries are 64 bits wide (their low words are read: the
+// reference's int64 table as it lies, where a conversion to 32 bits was a launch of its own, 3.4 to 5
+// us of every call).
 template <int EPL>
 LSK_DEV void route_select(const void* __restrict__ g, int gdt, int64_t ldg, int t, int E, int k, int renorm,
                           const int32_t* __restrict__ tab, int& e_mine, int& s_mine, int& S) {
@@ -42,7 +51,7 @@ LSK_DEV void route_select(const void* __restrict__ g, int gdt, int64_t ldg, int 
       int sc = 0;
       if (v < 1073741824.0f) {  // d < 16 << 26 (also false for NaN / inf)
         const int d = v > 0.0f ? (int)v : 0;
-        sc = tab[(d >> 13) & 8191] >> (d >> 26);
+        sc = tab[((d >> 13) & 8191) << (renorm >> 1)] >> (d >> 26);
       }
       s_all += sc;
       key[j] = ((uint32_t)sc << 16) | (uint32_t)(0xffff - e);
@@ -68,7 +77,7 @@ LSK_DEV void route_select(const void* __restrict__ g, int gdt, int64_t ldg, int 
     for (int j = 0; j < EPL; ++j)
       if (lane + 64 * j == e) key[j] = 0;
   }
-  S = renorm ? s_sum : s_all;
+  S = (renorm & 1) ? s_sum : s_all;
   S = S < 1 ? 1 : S;
 }
 

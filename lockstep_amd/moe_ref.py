@@ -311,10 +311,10 @@ def _route_fields(x, route):
         gd, code = g.contiguous(), L.LSK_BF16
     else:
         gd, code = g.to(torch.float32).contiguous(), L.LSK_F32
-    tb = ops.tab_i32(tab)
+    tb, flag = ops.router_tab(tab)
     idx = torch.empty((T, int(k)), dtype=torch.int64, device=x.device)
     w = torch.empty((T, int(k)), dtype=BF, device=x.device)
-    fields = dict(logits=gd.data_ptr(), logits_dtype=code, renormalize=1 if renormalize else 0, ld_logits=gd.shape[1],
+    fields = dict(logits=gd.data_ptr(), logits_dtype=code, renormalize=(1 if renormalize else 0) | flag, ld_logits=gd.shape[1],
                   router_tab=tb.data_ptr(), idx_out=idx.data_ptr(), w_out=w.data_ptr())
     return idx, w, fields, (gd, tb)
 

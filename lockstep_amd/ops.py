@@ -429,6 +429,14 @@ def tab_i32(tab: torch.Tensor) -> torch.Tensor:
     return tab.to(torch.int32).contiguous()
 
 
+def router_tab(tab: torch.Tensor):
+    """A caller's router table as the router kernels read it, with the flag for renormalize: the
+    reference's int64 table in place, any other type as int32."""
+    if tab.dtype == torch.int64 and tab.is_contiguous() and tab.numel() == 8192 and tab.is_cuda:
+        return tab, L.LSK_ROUTE_TAB64
+    return tab_i32(tab), 0
+
+
 def act(g: torch.Tensor, u, op: int) -> torch.Tensor:
     """Elementwise table activation in binary32 (shape of g)."""
     L.require_cuda(g, u, what="activation")
@@ -474,7 +482,8 @@ def router_topk(g: torch.Tensor, k: int, renormalize: bool, tab: torch.Tensor):
     idx = torch.empty((T, k), dtype=torch.int64, device=g.device)
     w = torch.empty((T, k), dtype=torch.bfloat16, device=g.device)
     if T:
-        L.call("lsk_router_topk", L.ptr(gd), code, E, T, E, int(k), 1 if renormalize else 0, L.ptr(tab_i32(tab)),
+        tb, flag = router_tab(tab)
+        L.call("lsk_router_topk", L.ptr(gd), code, E, T, E, int(k), (1 if renormalize else 0) | flag, L.ptr(tb),
                L.ptr(idx), L.ptr(w), L.stream_of(g))
     return idx, w
 
