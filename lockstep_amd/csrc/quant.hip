@@ -390,13 +390,51 @@ __global__ __launch_bounds__(256) void dyn_quant_pair_kernel(const float* __rest
 // rows of a pair) and its load four 256-byte runs of x (a chunk of each row of the pair, twice).
 // Every load of a step is issued before any is used, none under a branch (a lane past the run
 // re-reads the run's first float4 and stores nothing).
+// STAGE 0: as above.  A tensor of kSpecBytes and more is quantised on a guessed exponent instead, so
+// that x is read once where the guess holds (dyn_sample_kernel takes the maximum of 1 row in 32, and
+// the guess allows for a whole maximum 9% above it): STAGE 1 derives the exponent from the sample's
+// maxima, quantises, and leaves its run's own maximum in own[blockIdx.x] and the exponent in *guess;
+// STAGE 2 reduces those maxima, writes the tensor's exponent and returns, or, where the guess was
+// another, quantises again.  (MI355X, 8192 x 18944 binary32: maxima + quantise 97 + 138 us; sample +
+// STAGE 1 + 2 with the guess right 159, wrong 290.  On N(0,1) the maximum of 1 row in 32 is 0.88 of
+// the whole, so one scale in twelve guesses wrong: 170 us on average.)
 constexpr int kDynU2 = 8;
+constexpr int64_t kSpecBytes = 64 << 20;  // 117 MB: 45 us as two passes, 33 guessed; below, the launches cost what it saves
+constexpr int kSpecSamples = 512;
+constexpr float kSpecHeadroom = 1.09f;
 
-template <bool NT>
+// The maximum of rows 0, 32, 64, ... (whole rows: every column, and the first row, where activations
+// have their largest values), kSpecSamples partial maxima.
+__global__ __launch_bounds__(256) void dyn_sample_kernel(const float* __restrict__ x, int64_t M, int64_t K,
+                                                         float* __restrict__ out) {
+  __shared__ float red[4];
+  const int k4 = (int)(K >> 2);
+  const int64_t n = (M + 31) / 32 * k4;
+  float am = 0.0f;
+  constexpr int U = 4;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)kSpecSamples * 256 * U) {
+    float4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t j = i + (int64_t)u * kSpecSamples * 256;
+      const int64_t f = j < n ? j : i;
+      const int64_t r = f / k4;
+      v[u] = ((const float4*)(x + r * 32 * K))[f - r * k4];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      am = fmaxf(am, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
+  }
+  am = block_max<256>(am, red);
+  if (threadIdx.x == 0) out[blockIdx.x] = am;
+}
+
+template <bool NT, int STAGE = 0>
 __global__ __launch_bounds__(256) void dyn_quant_pair_flat_kernel(const float* __restrict__ x, int64_t M, int64_t K,
                                                                   const float* __restrict__ partial, int nparts,
                                                                   int8_t* __restrict__ q, int32_t* __restrict__ e_out,
-                                                                  int32_t* __restrict__ erow) {
+                                                                  int32_t* __restrict__ erow,
+                                                                  float* __restrict__ own, int32_t* __restrict__ guess) {
   __shared__ float red[4];
   const int n4 = (int)((M * K) >> 2);
   const int per = (n4 + (int)gridDim.x - 1) / (int)gridDim.x;
@@ -433,22 +471,39 @@ __global__ __launch_bounds__(256) void dyn_quant_pair_flat_kernel(const float* _
   // the first step requested before the partial maxima are reduced (it does not depend on them)
   float4 v[kDynU2];
   int f = f0;
-  if (b0 < b1) {
+  auto first = [&]() {
     addrs();
 #pragma unroll
     for (int u = 0; u < kDynU2; ++u) v[u] = load(src(f + 256 * u, lp[u], lr[u]));
-  }
+  };
+  if (STAGE != 2 && b0 < b1) first();
   float am = 0.0f;
   for (int j = threadIdx.x; j < nparts; j += 256) am = fmaxf(am, partial[j]);
   am = block_max<256>(am, red);
-  const int e = pow2_exponent(am);
+  const int e = pow2_exponent(STAGE == 1 ? f32_mul(am, kSpecHeadroom) : am);
   const float sc = pow2f(e);
-  if (blockIdx.x == 0 && threadIdx.x == 0) e_out[0] = e;
-  if (erow)
-    for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < M; r += (int64_t)gridDim.x * 256) erow[r] = e;
-  if (b0 >= b1) return;
+  if constexpr (STAGE == 1) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *guess = e;
+  } else {
+    if (blockIdx.x == 0 && threadIdx.x == 0) e_out[0] = e;
+    if (erow)
+      for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < M; r += (int64_t)gridDim.x * 256) erow[r] = e;
+  }
+  if constexpr (STAGE == 2) {
+    if (*guess == e) return;
+    if (b0 < b1) first();
+  }
+  float mine = 0.0f;
+  auto run_max = [&]() {
+    if constexpr (STAGE == 1) {
+#pragma unroll
+      for (int u = 0; u < kDynU2; ++u)
+        mine = fmaxf(mine, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
+    }
+  };
   uint32_t* q4 = (uint32_t*)q;
-  for (;;) {
+  for (; f < b1;) {
+    run_max();  // (a lane past the run holds the run's first float4)
 #pragma unroll
     for (int u = 0; u < kDynU2; ++u)
       if (f + 256 * u < b1) q4[f + 256 * u] = quant_pow2_x4(v[u], sc);
@@ -457,6 +512,10 @@ __global__ __launch_bounds__(256) void dyn_quant_pair_flat_kernel(const float* _
     addrs();
 #pragma unroll
     for (int u = 0; u < kDynU2; ++u) v[u] = load(src(f + 256 * u, lp[u], lr[u]));
+  }
+  if constexpr (STAGE == 1) {
+    mine = block_max<256>(mine, red);
+    if (threadIdx.x == 0) own[blockIdx.x] = mine;
   }
 }
 
@@ -638,21 +697,33 @@ int launch_quant8_dyn_pair(const float* x, int64_t M, int64_t K, int64_t ldx, in
   int64_t blocks = flat ? (total + 256 * 16 - 1) / (256 * 16) : M;
   blocks = blocks < 1 ? 1 : (blocks > kDynBlocks ? kDynBlocks : blocks);
   const bool nt = g_dynq != 2;
+  const bool in_order = g_dynq && flat && ldq == K && K % 64 == 0 && M % 2 == 0 && total < (int64_t)1 << 31 &&
+                        ((uintptr_t)q % 4) == 0;
+  int64_t fb = (total / 4 + 256 * kDynU2 * 2 - 1) / (256 * kDynU2 * 2);
+  fb = fb < 1 ? 1 : (fb > kDynBlocks ? kDynBlocks : fb);
+  if (in_order && g_dynq == 1 && 4 * total >= kSpecBytes) {
+    float* sample = partial + kDynBlocks;
+    int32_t* guess = (int32_t*)(sample + kSpecSamples);
+    hipLaunchKernelGGL(dyn_sample_kernel, dim3(kSpecSamples), dim3(256), 0, s, x, M, K, sample);
+    hipLaunchKernelGGL((dyn_quant_pair_flat_kernel<true, 1>), dim3((unsigned)fb), dim3(256), 0, s, x, M, K,
+                       (const float*)sample, kSpecSamples, q, e_out, erow, partial, guess);
+    hipLaunchKernelGGL((dyn_quant_pair_flat_kernel<true, 2>), dim3((unsigned)fb), dim3(256), 0, s, x, M, K,
+                       (const float*)partial, (int)fb, q, e_out, erow, (float*)nullptr, guess);
+    return lsk::check_launch("dyn_quant_pair_flat_kernel");
+  }
   if (nt)
     hipLaunchKernelGGL(dyn_amax_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat, partial);
   else
     hipLaunchKernelGGL(dyn_amax_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat, partial);
   int rc = lsk::check_launch("dyn_amax_kernel");
   if (rc) return rc;
-  if (g_dynq && flat && ldq == K && K % 64 == 0 && M % 2 == 0 && total < (int64_t)1 << 31 && ((uintptr_t)q % 4) == 0) {
-    int64_t fb = (total / 4 + 256 * kDynU2 * 2 - 1) / (256 * kDynU2 * 2);
-    fb = fb < 1 ? 1 : (fb > kDynBlocks ? kDynBlocks : fb);
+  if (in_order) {
     if (nt)
       hipLaunchKernelGGL(dyn_quant_pair_flat_kernel<true>, dim3((unsigned)fb), dim3(256), 0, s, x, M, K,
-                         (const float*)partial, (int)blocks, q, e_out, erow);
+                         (const float*)partial, (int)blocks, q, e_out, erow, (float*)nullptr, (int32_t*)nullptr);
     else
       hipLaunchKernelGGL(dyn_quant_pair_flat_kernel<false>, dim3((unsigned)fb), dim3(256), 0, s, x, M, K,
-                         (const float*)partial, (int)blocks, q, e_out, erow);
+                         (const float*)partial, (int)blocks, q, e_out, erow, (float*)nullptr, (int32_t*)nullptr);
     return lsk::check_launch("dyn_quant_pair_flat_kernel");
   }
   int64_t qblocks = (M + 1) / 2;
@@ -671,7 +742,7 @@ LinDynWs lindyn_layout(int64_t M, int64_t K) {
   auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
   LinDynWs l;
   l.partial = 0;
-  l.erow = up((int64_t)kDynBlocks * 4);
+  l.erow = up((int64_t)(kDynBlocks + kSpecSamples + 1) * 4);  // the partial maxima, the sample's, the guess
   l.q = l.erow + up(M * 4);
   l.bytes = l.q + up(((M + 1) & ~(int64_t)1) * ((K + 63) / 64 * 64));
   return l;

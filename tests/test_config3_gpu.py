@@ -340,3 +340,38 @@ def test_linear_dyn_quant_pass_variants(T, N, K, scale):
     with np.errstate(over="ignore", invalid="ignore"):
         ref = C.dequant_pow2(C.gemm_int(q_ref[rows], W8.T.astype(np.int64)), e_ref + 5)
     assert np.array_equal(got[0][1].numpy()[rows].view(np.uint32), f32_bits(ref))
+
+
+@pytest.mark.parametrize("case", ["right", "above", "below", "zero sample", "all zero", "first row"])
+def test_linear_dyn_guessed_exponent(case):
+    """A tensor large enough to be quantised on an exponent guessed from every 32nd row: the guess
+    right, too small (the maximum in a row the sample leaves out, also over an otherwise zero tensor),
+    too large (the headroom crosses a power of two the maximum does not), and all zeros: exponent and
+    result equal to the two-pass quant's, the exponent to the oracle's."""
+    from lockstep_amd import _lib as L
+    from lockstep_amd import ref_block_v1 as RB
+    say("guessed exponent", case)
+    T, K, N = 2050, 8256, 256
+    g = torch.Generator(device=dev())
+    g.manual_seed(5)
+    x = torch.randn((T, K), generator=g, device=dev()).clamp_(-5.0, 5.0)
+    if case == "above":
+        x[33, 77] = -8.5
+    elif case == "below":
+        x[64, 5] = 7.9
+    elif case in ("zero sample", "all zero"):
+        x.zero_()
+        if case == "zero sample":
+            x[2049, K - 1] = 3e-5
+    elif case == "first row":
+        x[0, 9] = 900.0
+    W = torch.randint(-127, 128, (N, K), generator=g, device=dev(), dtype=torch.int8)
+    y, e = RB.linear_dyn(x, W.t(), 7)
+    L.call("lsk_quant8_dyn_variant", 0)
+    try:
+        y0, e0 = RB.linear_dyn(x, W.t(), 7)
+    finally:
+        L.call("lsk_quant8_dyn_variant", 1)
+    m = np.array([float(x.abs().max())], np.float32)
+    assert int(e.item()) == int(e0.item()) == (0 if case == "all zero" else int(C._e_from_max(m)[0]))
+    assert torch.equal(y.view(torch.int32), y0.view(torch.int32))
