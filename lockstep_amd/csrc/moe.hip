@@ -211,21 +211,26 @@ LSK_DEV void place_chunk(const int32_t* ids, const uint16_t* wts, int T, int k, 
     }
   }
   __syncthreads();
-  if (t < T && tid >= wlo && tid < whi) {  // (the rows of tokens wlo .. whi-1 of the chunk)
-    for (int j = 0; j < k; ++j) {
-      const int e = my[j];
+  // The rows of tokens wlo .. whi-1 of the chunk, 256 / (whi - wlo) threads a token, each with every
+  // so-many-th of its routes (whi - wlo divides 256): a route costs a chain of up to 8 + k LDS reads,
+  // which one thread per token ran k times over with three waves of four idle.
+  const int span = whi - wlo, tl = wlo + tid % span, ta = c0 + tl;
+  const int32_t* mine = ids + tl * k;
+  if (ta < T) {
+    for (int j = tid / span; j < k; j += 256 / span) {
+      const int e = mine[j];
       if (e < 0) continue;
-      int rank = __popc(mask[e * 8 + (tid >> 5)] & ((1u << (tid & 31)) - 1u));
-      for (int wd = 0; wd < (tid >> 5); ++wd) rank += __popc(mask[e * 8 + wd]);
+      int rank = __popc(mask[e * 8 + (tl >> 5)] & ((1u << (tl & 31)) - 1u));
+      for (int wd = 0; wd < (tl >> 5); ++wd) rank += __popc(mask[e * 8 + wd]);
       const int p = base[e] + rank;
       int slot = 0;  // rank of e among the token's experts, ascending
       for (int j2 = 0; j2 < k; ++j2) {
-        const int e2 = my[j2];
+        const int e2 = mine[j2];
         if (e2 >= 0 && e2 < e) ++slot;
       }
-      row_tok[p] = t;
-      row_dst[p] = t * k + slot;
-      row_w[p] = bf16_to_f32(wts[tid * k + j]);
+      row_tok[p] = ta;
+      row_dst[p] = ta * k + slot;
+      row_w[p] = bf16_to_f32(wts[tl * k + j]);
     }
   }
   __syncthreads();
