@@ -49,7 +49,7 @@ def w8a8_matmul(x, W8, ws, bias=None, out_dtype=None, rowchunk: int = 0):
     want64 = odt == torch.float64
     if not want64 and odt not in _OUT:
         raise TypeError("w8a8_matmul: out_dtype %s not supported" % odt)
-    x2 = x.reshape(-1, shp[-1])
+    x2 = x if len(shp) == 2 and shp[1] > 0 else x.reshape(-1, shp[-1])
     if x2.dtype not in (torch.float32, torch.bfloat16, torch.float16):
         x2 = x2.float()
     if x2.shape[0] == 0:
@@ -62,7 +62,7 @@ def w8a8_matmul(x, W8, ws, bias=None, out_dtype=None, rowchunk: int = 0):
     y = ops.w8a8_matmul(x2, w, ws, bias, L.EPI_V21, L.LSK_F32 if want64 else _OUT[odt], w_pairs=wp)
     if want64:
         y = y.to(torch.float64)       # exact widening of the binary32 result
-    return y.reshape(*shp[:-1], N)
+    return y if len(shp) == 2 else y.reshape(*shp[:-1], N)
 
 
 def outlier_side(ho, wo):

@@ -13,7 +13,7 @@ from . import _lib as L
 
 def _rows(x: torch.Tensor) -> torch.Tensor:
     """x [..., K] -> a 2-D view/copy [rows, K] with unit stride along K."""
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 and x.shape[1] > 0 else x.reshape(-1, x.shape[-1])
     if x2.shape[-1] > 0 and x2.stride(-1) != 1:
         x2 = x2.contiguous()
     return x2
@@ -31,7 +31,8 @@ def weight_nk(b8: torch.Tensor) -> torch.Tensor:
 def _f32(t):
     if t is None:
         return None
-    t = t.to(torch.float32)
+    if t.dtype != torch.float32:
+        t = t.to(torch.float32)
     return t if t.is_contiguous() else t.contiguous()
 
 
@@ -107,9 +108,7 @@ def w8a8_matmul(x2: torch.Tensor, w_nk: torch.Tensor, ws: torch.Tensor, bias, or
     x2 = _rows(x2)
     M, K = x2.shape
     N = w_nk.shape[0]
-    tdt = {L.LSK_F32: torch.float32, L.LSK_BF16: torch.bfloat16, L.LSK_F16: torch.float16,
-           L.LSK_BF16_AS_F32: torch.float32}[out_dtype]
-    out = torch.empty((M, N), dtype=tdt, device=x2.device)
+    out = torch.empty((M, N), dtype=_OUT_T[out_dtype], device=x2.device)
     if M == 0 or N == 0:
         return out
     lib = L.load()
