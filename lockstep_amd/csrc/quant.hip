@@ -268,20 +268,72 @@ LSK_DEV uint32_t quant_pow2_x4(float4 v, float sc) {
          ((uint32_t)(uint8_t)quant_pow2_one(v.z, sc) << 16) | ((uint32_t)(uint8_t)quant_pow2_one(v.w, sc) << 24);
 }
 
+// The quantise passes' STAGE 0 derives the exponent from every block's maximum.  A contiguous tensor
+// of kSpecBytes and more is quantised on a guessed exponent instead, so
+// that x is read once where the guess holds (dyn_sample_kernel takes the maximum of 1 row in 32, and
+// the guess allows for a whole maximum 9% above it): STAGE 1 derives the exponent from the sample's
+// maxima, quantises, and leaves its run's own maximum in own[blockIdx.x] and the exponent in *guess;
+// STAGE 2 reduces those maxima, writes the tensor's exponent and returns, or, where the guess was
+// another, quantises again.  (MI355X, us, 8192 x 18944 binary32: maxima + quantise 97 + 138; sample + STAGE
+// 1 + 2 with the guess right 154, wrong 289.  On N(0,1) the maximum of 1 row in 32 is about 0.88 of
+// the whole, so with the headroom few scales guess wrong.)
+constexpr int64_t kSpecBytes = 64 << 20;  // (69 MB: 34 us as two passes, 24 guessed, 39 guessed wrong; not measured below)
+constexpr int kSpecSamples = 512;
+constexpr float kSpecHeadroom = 1.09f;
+
+// The maximum of rows 0, 32, 64, ... (whole rows: every column, and the first row, where activations
+// have their largest values), kSpecSamples partial maxima.
+__global__ __launch_bounds__(256) void dyn_sample_kernel(const float* __restrict__ x, int64_t M, int64_t K,
+                                                         float* __restrict__ out) {
+  __shared__ float red[4];
+  const int k4 = (int)(K >> 2);
+  const int64_t n = (M + 31) / 32 * k4;
+  float am = 0.0f;
+  constexpr int U = 4;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)kSpecSamples * 256 * U) {
+    float4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t j = i + (int64_t)u * kSpecSamples * 256;
+      const int64_t f = j < n ? j : i;
+      const int64_t r = f / k4;
+      v[u] = ((const float4*)(x + r * 32 * K))[f - r * k4];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      am = fmaxf(am, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
+  }
+  am = block_max<256>(am, red);
+  if (threadIdx.x == 0) out[blockIdx.x] = am;
+}
+
+template <int STAGE = 0>
 __global__ __launch_bounds__(256) void dyn_quant_kernel(const float* __restrict__ x, int64_t M, int64_t K,
                                                         int64_t ldx, int flat, const float* __restrict__ partial,
                                                         int nparts, int8_t* __restrict__ q, int64_t ldq,
-                                                        int32_t* __restrict__ e_out, int32_t* __restrict__ erow) {
+                                                        int32_t* __restrict__ e_out, int32_t* __restrict__ erow,
+                                                        float* __restrict__ own, int32_t* __restrict__ guess) {
   __shared__ float red[4];
   float am = 0.0f;
   for (int j = threadIdx.x; j < nparts; j += 256) am = fmaxf(am, partial[j]);
   am = block_max<256>(am, red);
-  const int e = pow2_exponent(am);   // 0 for an all-zero tensor, whose q is then 0 as well
+  // 0 for an all-zero tensor, whose q is then 0 as well
+  const int e = pow2_exponent(STAGE == 1 ? f32_mul(am, kSpecHeadroom) : am);
   const float sc = pow2f(e);         // e in [-32, 40]: a normal power of two
   const int64_t stride = (int64_t)gridDim.x * 256;
-  if (blockIdx.x == 0 && threadIdx.x == 0) e_out[0] = e;
-  if (erow)
-    for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < M; r += stride) erow[r] = e;
+  if constexpr (STAGE == 1) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *guess = e;
+  } else {
+    if (blockIdx.x == 0 && threadIdx.x == 0) e_out[0] = e;
+    if (erow)
+      for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < M; r += stride) erow[r] = e;
+  }
+  if (STAGE == 2 && *guess == e) return;
+  float mine = 0.0f;
+  auto see = [&](const float4& v) {
+    if constexpr (STAGE == 1)
+      mine = fmaxf(mine, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+  };
   if (flat) {
     // pairs of float4 (eight elements, one 8-byte store of q), each block a contiguous run
     const int64_t n8 = (M * K) >> 3;
@@ -298,15 +350,27 @@ __global__ __launch_bounds__(256) void dyn_quant_kernel(const float* __restrict_
         v[u][1] = ld_nt(x4 + 2 * (i + 256 * u) + 1);
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+      for (int u = 0; u < U; ++u) {
+        see(v[u][0]);
+        see(v[u][1]);
         *(v2u32*)(q + 8 * (i + 256 * u)) = v2u32{quant_pow2_x4(v[u][0], sc), quant_pow2_x4(v[u][1], sc)};
+      }
     }
     for (; i < b1; i += 256) {
       const float4 a = ld_nt(x4 + 2 * i), b = ld_nt(x4 + 2 * i + 1);
+      see(a);
+      see(b);
       *(v2u32*)(q + 8 * i) = v2u32{quant_pow2_x4(a, sc), quant_pow2_x4(b, sc)};
     }
     if (blockIdx.x == gridDim.x - 1)
-      for (int64_t j = (n8 << 3) + threadIdx.x; j < M * K; j += 256) q[j] = quant_pow2_one(x[j], sc);
+      for (int64_t j = (n8 << 3) + threadIdx.x; j < M * K; j += 256) {
+        if (STAGE == 1) mine = fmaxf(mine, fabsf(x[j]));
+        q[j] = quant_pow2_one(x[j], sc);
+      }
+    if constexpr (STAGE == 1) {
+      mine = block_max<256>(mine, red);
+      if (threadIdx.x == 0) own[blockIdx.x] = mine;
+    }
   } else {
     for (int64_t r = blockIdx.x; r < M; r += gridDim.x)
       for (int64_t c = threadIdx.x; c < K; c += 256) q[r * ldq + c] = quant_pow2_one(x[r * ldx + c], sc);
@@ -390,45 +454,7 @@ __global__ __launch_bounds__(256) void dyn_quant_pair_kernel(const float* __rest
 // rows of a pair) and its load four 256-byte runs of x (a chunk of each row of the pair, twice).
 // Every load of a step is issued before any is used, none under a branch (a lane past the run
 // re-reads the run's first float4 and stores nothing).
-// STAGE 0: as above.  A tensor of kSpecBytes and more is quantised on a guessed exponent instead, so
-// that x is read once where the guess holds (dyn_sample_kernel takes the maximum of 1 row in 32, and
-// the guess allows for a whole maximum 9% above it): STAGE 1 derives the exponent from the sample's
-// maxima, quantises, and leaves its run's own maximum in own[blockIdx.x] and the exponent in *guess;
-// STAGE 2 reduces those maxima, writes the tensor's exponent and returns, or, where the guess was
-// another, quantises again.  (MI355X, 8192 x 18944 binary32: maxima + quantise 97 + 138 us; sample +
-// STAGE 1 + 2 with the guess right 159, wrong 290.  On N(0,1) the maximum of 1 row in 32 is 0.88 of
-// the whole, so one scale in twelve guesses wrong: 170 us on average.)
 constexpr int kDynU2 = 8;
-constexpr int64_t kSpecBytes = 64 << 20;  // 117 MB: 45 us as two passes, 33 guessed; below, the launches cost what it saves
-constexpr int kSpecSamples = 512;
-constexpr float kSpecHeadroom = 1.09f;
-
-// The maximum of rows 0, 32, 64, ... (whole rows: every column, and the first row, where activations
-// have their largest values), kSpecSamples partial maxima.
-__global__ __launch_bounds__(256) void dyn_sample_kernel(const float* __restrict__ x, int64_t M, int64_t K,
-                                                         float* __restrict__ out) {
-  __shared__ float red[4];
-  const int k4 = (int)(K >> 2);
-  const int64_t n = (M + 31) / 32 * k4;
-  float am = 0.0f;
-  constexpr int U = 4;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)kSpecSamples * 256 * U) {
-    float4 v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t j = i + (int64_t)u * kSpecSamples * 256;
-      const int64_t f = j < n ? j : i;
-      const int64_t r = f / k4;
-      v[u] = ((const float4*)(x + r * 32 * K))[f - r * k4];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      am = fmaxf(am, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
-  }
-  am = block_max<256>(am, red);
-  if (threadIdx.x == 0) out[blockIdx.x] = am;
-}
-
 template <bool NT, int STAGE = 0>
 __global__ __launch_bounds__(256) void dyn_quant_pair_flat_kernel(const float* __restrict__ x, int64_t M, int64_t K,
                                                                   const float* __restrict__ partial, int nparts,
@@ -626,17 +652,29 @@ __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* __restrict__ p,
 }
 
 // Launches of quant8_dyn on a workspace of kDynBlocks floats.
+// spec: partial has room for the sample's maxima and the guess behind the blocks' maxima (linear_dyn's
+// workspace), so a large contiguous tensor is quantised on a guessed exponent.
 int launch_quant8_dyn(const float* x, int64_t M, int64_t K, int64_t ldx, int8_t* q, int64_t ldq, int32_t* e_out,
-                      int32_t* erow, float* partial, hipStream_t s) {
+                      int32_t* erow, float* partial, bool spec, hipStream_t s) {
   const int64_t total = M * K;
   const int flat = (ldx == K && ldq == K && ((uintptr_t)x % 16) == 0 && ((uintptr_t)q % 8) == 0) ? 1 : 0;
   int64_t blocks = flat ? (total + 256 * 16 - 1) / (256 * 16) : M;
   blocks = blocks < 1 ? 1 : (blocks > kDynBlocks ? kDynBlocks : blocks);
+  if (spec && flat && K % 4 == 0 && 4 * total >= kSpecBytes) {
+    float* sample = partial + kDynBlocks;
+    int32_t* guess = (int32_t*)(sample + kSpecSamples);
+    hipLaunchKernelGGL(dyn_sample_kernel, dim3(kSpecSamples), dim3(256), 0, s, x, M, K, sample);
+    hipLaunchKernelGGL(dyn_quant_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat,
+                       (const float*)sample, kSpecSamples, q, ldq, e_out, erow, partial, guess);
+    hipLaunchKernelGGL(dyn_quant_kernel<2>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat,
+                       (const float*)partial, (int)blocks, q, ldq, e_out, erow, (float*)nullptr, guess);
+    return lsk::check_launch("dyn_quant_kernel");
+  }
   hipLaunchKernelGGL(dyn_amax_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat, partial);
   int rc = lsk::check_launch("dyn_amax_kernel");
   if (rc) return rc;
-  hipLaunchKernelGGL(dyn_quant_kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat,
-                     (const float*)partial, (int)blocks, q, ldq, e_out, erow);
+  hipLaunchKernelGGL(dyn_quant_kernel<0>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat,
+                     (const float*)partial, (int)blocks, q, ldq, e_out, erow, (float*)nullptr, (int32_t*)nullptr);
   return lsk::check_launch("dyn_quant_kernel");
 }
 
@@ -853,7 +891,7 @@ extern "C" int lsk_linear_dyn(const float* x, int64_t M, int64_t K, int64_t ldx,
   const int64_t ldq = pair ? kp : (K + 15) / 16 * 16;
   if (stages & 1) {
     const int rc = pair ? launch_quant8_dyn_pair(x, M, K, ldx, q, ldq, ex_out, erow, partial, s)
-                        : launch_quant8_dyn(x, M, K, ldx, q, ldq, ex_out, erow, partial, s);
+                        : launch_quant8_dyn(x, M, K, ldx, q, ldq, ex_out, erow, partial, g_dynq == 1, s);
     if (rc) return rc;
   }
   if (!(stages & 2) || M == 0 || N == 0) return LSK_OK;
@@ -885,7 +923,7 @@ extern "C" int lsk_quant8_dyn(const float* x, int64_t M, int64_t K, int64_t ldx,
               "lsk_quant8_dyn: workspace of %lld bytes required (%lld given)", (long long)lsk_quant8_dyn_workspace(),
               (long long)workspace_bytes);
   LSK_REQUIRE(M * K == 0 || (x && q), "lsk_quant8_dyn: null pointer");
-  return launch_quant8_dyn(x, M, K, ldx, q, ldq, e_out, erow_out, (float*)workspace, (hipStream_t)stream);
+  return launch_quant8_dyn(x, M, K, ldx, q, ldq, e_out, erow_out, (float*)workspace, false, (hipStream_t)stream);
 }
 
 extern "C" int lsk_rowquant(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, int8_t* q,
@@ -935,7 +973,7 @@ extern "C" int lsk_quant8_pow2(const float* x, int64_t M, int64_t K, int64_t ldx
   if (mode == 0) {
     // the workspace (4 * (M + K + 64) bytes) holds the partial maxima of every grid quant8_dyn
     // launches for this size
-    return launch_quant8_dyn(x, M, K, ldx, q, ldq, e_out, nullptr, (float*)workspace, s);
+    return launch_quant8_dyn(x, M, K, ldx, q, ldq, e_out, nullptr, (float*)workspace, false, s);
   }
   uint32_t* amax = (uint32_t*)workspace;
   if (K > 0) {

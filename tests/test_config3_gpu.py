@@ -342,8 +342,9 @@ def test_linear_dyn_quant_pass_variants(T, N, K, scale):
     assert np.array_equal(got[0][1].numpy()[rows].view(np.uint32), f32_bits(ref))
 
 
+@pytest.mark.parametrize("T,K,N", [(2050, 8256, 256), (1025, 16496, 256)])   # row pairs / rows (K-split tiles)
 @pytest.mark.parametrize("case", ["right", "above", "below", "zero sample", "all zero", "first row"])
-def test_linear_dyn_guessed_exponent(case):
+def test_linear_dyn_guessed_exponent(case, T, K, N):
     """A tensor large enough to be quantised on an exponent guessed from every 32nd row: the guess
     right, too small (the maximum in a row the sample leaves out, also over an otherwise zero tensor),
     too large (the headroom crosses a power of two the maximum does not), and all zeros: exponent and
@@ -351,7 +352,6 @@ def test_linear_dyn_guessed_exponent(case):
     from lockstep_amd import _lib as L
     from lockstep_amd import ref_block_v1 as RB
     say("guessed exponent", case)
-    T, K, N = 2050, 8256, 256
     g = torch.Generator(device=dev())
     g.manual_seed(5)
     x = torch.randn((T, K), generator=g, device=dev()).clamp_(-5.0, 5.0)
@@ -362,7 +362,7 @@ def test_linear_dyn_guessed_exponent(case):
     elif case in ("zero sample", "all zero"):
         x.zero_()
         if case == "zero sample":
-            x[2049, K - 1] = 3e-5
+            x[(T - 2) // 32 * 32 + 1, K - 1] = 3e-5
     elif case == "first row":
         x[0, 9] = 900.0
     W = torch.randint(-127, 128, (N, K), generator=g, device=dev(), dtype=torch.int8)
