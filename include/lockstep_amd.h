@@ -200,6 +200,14 @@ int lsk_planes_linear(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_
                       const int8_t* w, int64_t ldw, int64_t N, int wbits, const float* ws, const float* bias, void* out,
                       int out_dtype, int64_t ldo, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* lsk_planes_linear with w_pairs (NULL, or lsk_pack_row_pairs of the stacked planes w [Pw * N, K]),
+ * read where the stacked activation planes run on the skinny decode GEMV (lsk_gemm_reads_row_pairs of
+ * Pa * M rows, at most 32, and Pw * N channels).  The same results. */
+int lsk_planes_linear_pairs(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int abits,
+                            const float* sdiv, const int8_t* w, int64_t ldw, const int8_t* w_pairs, int64_t N, int wbits,
+                            const float* ws, const float* bias, void* out, int out_dtype, int64_t ldo, void* workspace,
+                            int64_t workspace_bytes, void* stream);
+
 /* ---------------------------------------------------------------- the contract 2.6 float norm */
 
 /* The float RMSNorm (replaces t16n_ref.rmsnorm_float / row_sum_float, reference/t16n_ref.py:53-92),
@@ -276,8 +284,9 @@ int lsk_quant8_dyn_single_pass(int on);
 /* Tuning control with no counterpart in the reference: the quantise pass of lsk_linear_dyn's
  * quant8_dyn (0: row pairs per block; 1, the default: a contiguous tensor with K % 64 == 0 and M
  * even walked in the order of q, a wave's stores covering two whole 128-byte lines of q, 0
- * otherwise; 2: as 1 with ordinary rather than non-temporal loads in both passes).  The same
- * exponent and q.  Thread-local. */
+ * otherwise; from 64 MB of x the exponent guessed from every 32nd row and the pass repeated only if
+ * the whole maximum says otherwise; 2: as 1 without the guess and with ordinary rather than
+ * non-temporal loads in both passes).  The same exponent and q.  Thread-local. */
 int lsk_quant8_dyn_variant(int v);
 
 /* Tuning control with no counterpart in the reference: the persistent form of the 256x256
@@ -313,8 +322,8 @@ int lsk_quant8_dyn(const float* x, int64_t M, int64_t K, int64_t ldx, int8_t* q,
  * erow, shift = ew, binary32 out), bit for bit.  x [M, K] binary32 (row stride ldx); w [N, K] int8
  * (row stride ldw); y [M, N] binary32 (row stride ldy); ex_out[0] = ex.  q stays in the workspace
  * (lsk_linear_dyn_workspace(M, K) bytes, 256-byte aligned), written in the layout the GEMM tiles
- * read fastest (rows paired by 64-byte K chunks when every tile is a ping-pong tile).  Three
- * launches, nothing to clear beforehand (graph-capturable).  w_pairs: null, or the same weight in
+ * read fastest (rows paired by 64-byte K chunks when every tile is a ping-pong tile).  Three to
+ * five launches, nothing to clear beforehand (graph-capturable).  w_pairs: null, or the same weight in
  * the row-pair layout (lsk_pack_row_pairs), which the GEMM then reads when q takes that layout.
  * stages: 3 the whole site; 1 only the quant (q and the exponents into the workspace, ex_out), 2
  * only the GEMM from a workspace that a stage-1 call with the same arguments filled (to time the
@@ -659,7 +668,9 @@ int lsk_moe_pp_skinny_rows(int rows);
 
 /* Tuning control with no counterpart in the reference: the main loop of the grouped MXFP4
  * expert GEMMs (0: direct-to-LDS operand staging with fp4 fragments converted per wave, a
- * two-stage ring, three blocks per CU, the default; 1: register-staged operands converted to bf16
+ * two-stage ring, three blocks per CU, the default, and for MXFP4 layers with per-row activation
+ * scales past the skinny GEMM the block-scaled MFMA on six-bit activation planes, given exponent
+ * bytes in 16 .. 239, mx_safe 0 and act_tab; 1: register-staged operands converted to bf16
  * before LDS; 2: as 0 with a three-stage ring and two blocks per CU; 3: as 0, with the skinny
  * grouped MX GEMM -- an expert's rows 16 at a time in LDS, the codes streamed into the bf16 MFMA --
  * wherever the layer can take it, which 0 does by size: MXFP4 layers with per-row activation

@@ -17,11 +17,10 @@
 namespace lsk {
 int launch_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, int64_t M, int64_t N, int64_t K,
                 const EpiParams& ep, hipStream_t s);
+bool gemm_takes_skinny(const int8_t* w, int64_t ldw, int64_t M, int64_t N, int64_t K, int64_t lda);
 }  // namespace lsk
 
 namespace {
-
-constexpr float kAmaxFloor = 0x1.5798eep-27f;  // binary32 nearest 1e-8 (torch clamp(min=1e-8))
 
 // The element the quantiser sees: x, or fl32(x / sdiv[k]) (op 1, the runtime SmoothQuant
 // divide) or fl32(x * sdiv[k]) (op 2, the prepare-time weight fold).
@@ -29,18 +28,6 @@ LSK_DEV float col_op(float v, const float* sdiv, int op, int64_t k) {
   if (op == 1) return f32_div(v, sdiv[k]);
   if (op == 2) return f32_mul(v, sdiv[k]);
   return v;
-}
-
-template <int THREADS>
-LSK_DEV float block_max(float v, float* red) {
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  float r = red[0];
-  for (int w = 1; w < THREADS / 64; ++w) r = fmaxf(r, red[w]);
-  __syncthreads();
-  return r;
 }
 
 // One block per row: amax (exact, order-free), asc = fl32(max(amax, 1e-8) / amax_q),
@@ -166,8 +153,13 @@ extern "C" int lsk_quant_planes(const void* x, int x_dtype, int64_t ldx, int64_t
   LSK_REQUIRE(asc && (q || q32) && (x || K == 0), "lsk_quant_planes: null pointer");
   LSK_REQUIRE(ldx >= K && (q32 || ldq >= K), "lsk_quant_planes: leading dimension below K");
   LSK_REQUIRE(M <= 0x7fffffff, "lsk_quant_planes: too many rows");
-  hipLaunchKernelGGL(quant_planes_kernel<256>, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, x, x_dtype, M, K,
-                     ldx, bits, sdiv, sdiv_op, q, ldq, q32, asc);
+  // few rows (the head's activations) are one row's latency: 16 waves a row (8 x 3584: 8.4 -> 4.8 us)
+  if (M <= 256)
+    hipLaunchKernelGGL(quant_planes_kernel<1024>, dim3((unsigned)M), dim3(1024), 0, (hipStream_t)stream, x, x_dtype, M,
+                       K, ldx, bits, sdiv, sdiv_op, q, ldq, q32, asc);
+  else
+    hipLaunchKernelGGL(quant_planes_kernel<256>, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, x, x_dtype, M, K,
+                       ldx, bits, sdiv, sdiv_op, q, ldq, q32, asc);
   return lsk::check_launch("quant_planes_kernel");
 }
 
@@ -211,6 +203,14 @@ extern "C" int lsk_planes_linear(const void* x, int x_dtype, int64_t ldx, int64_
                                  const float* sdiv, const int8_t* w, int64_t ldw, int64_t N, int wbits, const float* ws,
                                  const float* bias, void* out, int out_dtype, int64_t ldo, void* workspace,
                                  int64_t workspace_bytes, void* stream) {
+  return lsk_planes_linear_pairs(x, x_dtype, ldx, M, K, abits, sdiv, w, ldw, nullptr, N, wbits, ws, bias, out, out_dtype,
+                                 ldo, workspace, workspace_bytes, stream);
+}
+
+extern "C" int lsk_planes_linear_pairs(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int abits,
+                                       const float* sdiv, const int8_t* w, int64_t ldw, const int8_t* w_pairs, int64_t N,
+                                       int wbits, const float* ws, const float* bias, void* out, int out_dtype,
+                                       int64_t ldo, void* workspace, int64_t workspace_bytes, void* stream) {
   LSK_REQUIRE(M >= 0 && N >= 0 && K >= 0, "lsk_planes_linear: negative size");
   LSK_REQUIRE(bits_ok(abits) && bits_ok(wbits), "lsk_planes_linear: widths must be 8, 11 or 15");
   // every plane product is bounded by 128 * 128 * K; int32 is exact for K <= 131071
@@ -242,7 +242,13 @@ extern "C" int lsk_planes_linear(const void* x, int x_dtype, int64_t ldx, int64_
                               sdiv, sdiv ? 1 : 0, q, ldq, nullptr, asc + m0, stream);
     if (rc) return rc;
     EpiParams ep{LSK_EPI_RAW, LSK_I32, nullptr, nullptr, nullptr, nullptr, nullptr, 0, c, (int64_t)pw * N};
-    if ((rc = lsk::launch_gemm(q, ldq, w, ldw, (int64_t)pa * rows, (int64_t)pw * N, K, ep, s))) return rc;
+    // a decode batch's planes on the skinny GEMV: the planes' row-pair copy, read in whole lines
+    const int64_t kp = (K + 63) / 64 * 64;
+    const bool pairs = w_pairs && lsk::gemm_takes_skinny(w_pairs, kp, (int64_t)pa * rows, (int64_t)pw * N, K, ldq);
+    ep.pairs = pairs ? 2 : 0;
+    if ((rc = lsk::launch_gemm(q, ldq, pairs ? w_pairs : w, pairs ? kp : ldw, (int64_t)pa * rows, (int64_t)pw * N, K, ep,
+                               s)))
+      return rc;
     if ((rc = lsk_planes_combine(c, (int64_t)pw * N, rows, N, abits, wbits, asc + m0, ws, bias,
                                  (char*)out + m0 * ldo * osz, out_dtype, ldo, stream)))
       return rc;

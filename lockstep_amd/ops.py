@@ -219,8 +219,9 @@ def split_planes(a: torch.Tensor, sh: int):
 
 
 def planes_linear(x2: torch.Tensor, w2: torch.Tensor, wbits: int, ws: torch.Tensor, abits: int, sdiv=None,
-                  bias=None, out_dtype: int = L.LSK_F32) -> torch.Tensor:
-    """The a<abits>w<wbits> linear of rows x2 [M, K] against stacked weight planes w2 [P * N, K]."""
+                  bias=None, out_dtype: int = L.LSK_F32, w_pairs=None) -> torch.Tensor:
+    """The a<abits>w<wbits> linear of rows x2 [M, K] against stacked weight planes w2 [P * N, K];
+    w_pairs: None or planes_pairs(w2, M, abits)."""
     L.require_cuda(x2, w2, ws, sdiv, bias, what="planes_linear")
     _bits_ok(abits)
     _bits_ok(wbits)
@@ -238,10 +239,17 @@ def planes_linear(x2: torch.Tensor, w2: torch.Tensor, wbits: int, ws: torch.Tens
     nbytes = L.load().lsk_planes_linear_workspace(M, K, N, int(abits), int(wbits))
     work = torch.empty((nbytes,), dtype=torch.uint8, device=x2.device)
     ws, sdiv, bias = _f32(ws), _f32(sdiv), _f32(bias)
-    L.call("lsk_planes_linear", L.ptr(x2), xc, x2.stride(0) if M > 1 else max(K, 1), M, K, int(abits), L.ptr(sdiv),
-           L.ptr(w2), w2.stride(0) if w2.shape[0] > 1 else max(K, 1), N, int(wbits), L.ptr(ws), L.ptr(bias),
-           L.ptr(out), out_dtype, N, L.ptr(work), nbytes, L.stream_of(x2))
+    L.call("lsk_planes_linear_pairs", L.ptr(x2), xc, x2.stride(0) if M > 1 else max(K, 1), M, K, int(abits), L.ptr(sdiv),
+           L.ptr(w2), w2.stride(0) if w2.shape[0] > 1 else max(K, 1), L.ptr(w_pairs), N, int(wbits), L.ptr(ws),
+           L.ptr(bias), L.ptr(out), out_dtype, N, L.ptr(work), nbytes, L.stream_of(x2))
     return out
+
+
+def planes_pairs(w2: torch.Tensor, rows: int, abits: int):
+    """The stacked planes' row-pair copy (kept on w2, row_pairs_of) where the planes of `rows`
+    activation rows are a decode batch that reads it (at most 32), else None."""
+    n = int(rows) * (1 if abits == 8 else 2)
+    return row_pairs_of(w2, n) if n <= 32 and w2.dtype == torch.int8 else None
 
 
 def quant8_pow2(x: torch.Tensor, mode: int):

@@ -150,3 +150,23 @@ def test_int64_rounding_at_halfway_cases():
     y = v.logits(to_dev(x))
     want = np.array(targets, np.int64).astype(F32)[None, :]
     assert np.array_equal(bits(y), f32_bits(want))
+
+
+@pytest.mark.parametrize("spec", ["a15w15", "a8", "w15"])
+@pytest.mark.parametrize("M,N,K", [(3, 8200, 272), (16, 16385, 64), (17, 8192, 80), (40, 8192, 128)])
+def test_variant_logits_on_row_pairs(spec, M, N, K):
+    """Decode batches of a wide head read the planes' row-pair copy (up to 32 stacked rows; 34 and 80
+    read the planes): the same logits as the planes alone, before and after an in-place update of
+    them, whose copy is remade."""
+    from lockstep_amd import ops
+    from lockstep_amd import t16h_lmvariants as T
+    say("variant pairs", spec, M, N, K)
+    r = np.random.default_rng(M + N)
+    W = to_dev((r.standard_normal((N, K)) * 0.05).astype(np.float32))
+    x = to_dev(r.standard_normal((M, K)).astype(np.float32))
+    v = T.build(spec).prepare(W)
+    for step in range(2):
+        y = v.logits(x)
+        y0 = ops.planes_linear(x, v._w2, v.wbits, v.ws, v.abits)
+        assert torch.equal(y.view(torch.int32), y0.view(torch.int32)), step
+        v._w2.copy_(v._w2.flip(0).contiguous())
