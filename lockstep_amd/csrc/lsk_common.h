@@ -52,16 +52,6 @@ LSK_DEV uint32_t wave_reduce_dpp(uint32_t v, uint32_t ident, Op op) {
 LSK_DEV uint32_t wave_max_u32(uint32_t v) {
   return wave_reduce_dpp(v, 0u, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
 }
-// The maximum over each half of the wave, in its last lane (31 and 63; the other lanes hold partial
-// maxima).
-LSK_DEV uint32_t half_max_u32(uint32_t v) {
-  auto op = [](uint32_t a, uint32_t b) { return a > b ? a : b; };
-  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, false));   // quad [1,0,3,2]
-  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, false));   // quad [2,3,0,1]
-  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));  // half-row mirror
-  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false));  // row mirror
-  return op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row bcast 15
-}
 LSK_DEV int wave_sum_i32(int v) {
   return (int)wave_reduce_dpp((uint32_t)v, 0u, [](uint32_t a, uint32_t b) { return (uint32_t)((int)a + (int)b); });
 }

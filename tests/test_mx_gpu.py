@@ -412,10 +412,11 @@ def test_moe_mx_grouped_main_loops(mxv, big_exp):
 @pytest.mark.parametrize("act", ["silu", "swigluoai"])
 @pytest.mark.parametrize("T,E,k,H,I,bias,big", [(257, 4, 2, 96, 160, False, False), (600, 3, 2, 352, 224, True, False),
                                                 (300, 40, 1, 64, 32, True, False), (513, 5, 3, 288, 96, False, True),
-                                                (1200, 2, 1, 32, 128, True, True)])
+                                                (1200, 2, 1, 32, 128, True, True),
+                                                (25, 4, 2, 96, 160, True, False), (256, 5, 2, 160, 96, False, True)])
 def test_moe_mx_six_bit_tiles(act, T, E, k, H, I, bias, big):
-    """Layers past 256 tokens on the block-scaled MFMA tiles against the oracle: one to eleven MX
-    blocks (K stages of four), experts of no rows up to several 128-row tiles, empty and partial
+    """Layers past 256 tokens (past 24 where the skinny GEMM is turned down) on the block-scaled MFMA
+    tiles against the oracle: one to eleven MX blocks (K stages of four), experts of no rows up to several 128-row tiles, empty and partial
     32-row strips, partial column tiles, every int8 magnitude (a row of extreme values), gate values
     inside and outside the table's run in LDS, and with `big` the outermost exponent bytes these
     tiles take (16 and 239, which also turn the NaN-free epilogue off)."""
@@ -443,8 +444,9 @@ def test_moe_mx_six_bit_tiles(act, T, E, k, H, I, bias, big):
                      None if b2 is None else to_dev(b2)))
     tables = MR.ExpertTablesMX(dexp, packed=True)
     ridx, rw = routing_device(idx, w)
-    y, _, _ = MR.moe_forward_mx(bf16_dev(x), None, tables, k, True, _tab(), 0, getattr(MR, "act_" + act),
-                                routing=(ridx, rw))
+    with MR.kernel_choice(moe=0 if T <= 256 else None):
+        y, _, _ = MR.moe_forward_mx(bf16_dev(x), None, tables, k, True, _tab(), 0, getattr(MR, "act_" + act),
+                                    routing=(ridx, rw))
     with np.errstate(over="ignore", invalid="ignore"):
         ref = C.moe_forward_mx(x, oexp, idx, w, getattr(C, "act_" + act))
     assert np.array_equal(u16(y), ref), int((u16(y) != ref).sum())
