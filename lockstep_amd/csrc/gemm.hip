@@ -1974,22 +1974,30 @@ static int launch_mid(bool rows64, int S, const int8_t* a, int lda, const int8_t
 // (Before, with 128x128 register-staged tiles up to M = 128 and the 256-row tiles beyond, and after:
 // 3584 x 18944 at M = 72 / 300 / 500 151.7 / 107.2 / 124.9 -> 29.9 / 48.6 / 66.0; 4608 x 3584 at M =
 // 72 / 777 44.4 / 32.7 -> 17.3 / 28.0; 28672 x 4096 at M = 72 58.0 -> 37.7.)
+// The outlier epilogue (v25, past 32 rows) is per-block latency that grows with the tile's rows, and a
+// split moves it into the combine: 4 us more on 128-row tiles, 5.5 on a split, 8 on each round of 64-row
+// tiles past the first, and those at any M (whole call, 16 channels, 128-row or split / 64-row tiles: 4608 x 3584 at
+// M = 40 / 300 32.4 / 31.6 -> 24.0 / 25.7 us, 3584 x 3584 at M = 150 / 500 30.3 / 32.3 -> 24.4 / 25.8;
+// 4608 x 3584 at M = 500, two rounds, 32.0 / 42.9).
 struct MidPlan {
   bool rows64;
   int S;
 };
-static MidPlan mid_plan(int64_t M, int64_t N, int64_t K, int64_t part_bytes) {
+static MidPlan mid_plan(int64_t M, int64_t N, int64_t K, int64_t part_bytes, bool v25 = false) {
   MidPlan p{false, 0};
   if (M <= 16 || M > 2048 || (M > 128 && K < 1024) || (M + 127) / 128 * ((N + 127) / 128) > 256) return p;
   const bool gemv = M <= 32;
   if (gemv && (N * K < (15 << 20) || gemv_takes_skinny(M, N, K))) return p;
   const int64_t stages = (K + 127) / 128;
   double best = 1e30;
-  for (int r64 = M <= 256 ? 1 : 0; r64 >= 0; --r64) {
+  const bool side = v25 && !gemv;
+  for (int r64 = M <= 256 || side ? 1 : 0; r64 >= 0; --r64) {
     const int64_t t = (M + (r64 ? 63 : 127)) / (r64 ? 64 : 128) * ((N + 127) / 128);
     for (int S = 1; S == 1 || (S <= 16 && t * S <= 256 && stages >= 4 * S && split_bytes(M, N, S) <= part_bytes); ++S) {
-      const double us = (r64 ? 0.38 : 0.45) * (double)((stages + S - 1) / S) * (double)((t * S + 255) / 256) +
-                        (S > 1 ? 4.5 + 8e-6 / 6 * (double)(S * M * N) : 0.0);
+      const double rounds = (double)((t * S + 255) / 256);
+      const double us = (r64 ? 0.38 : 0.45) * (double)((stages + S - 1) / S) * rounds +
+                        (S > 1 ? 4.5 + 8e-6 / 6 * (double)(S * M * N) : 0.0) +
+                        (side ? S > 1 ? 5.5 : r64 ? 8.0 * (rounds - 1.0) : 4.0 : 0.0);
       if (us < best) best = us, p.rows64 = r64 != 0, p.S = S;
     }
   }
@@ -2044,7 +2052,7 @@ int launch_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, int6
     return launch_mid(g_force_tile == 20, fits ? g_split : 1, a, (int)lda, w, (int)ldw, iM, iN, iK, ep, s);
   }
   if (g_force_tile < 0 && ep.pairs == 0) {
-    const MidPlan p = mid_plan(M, N, K, ep.part_bytes);
+    const MidPlan p = mid_plan(M, N, K, ep.part_bytes, ep.order == LSK_EPI_V25);
     if (p.S > 0) return launch_mid(p.rows64, p.S, a, (int)lda, w, (int)ldw, iM, iN, iK, ep, s);
   }
   if (M <= 32 && (g_force_tile < 0 || g_force_tile == 5)) {

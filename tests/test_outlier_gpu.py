@@ -162,3 +162,17 @@ def test_outlier_tile_epilogues(tile, M, N, K, ko):
         L.call("lsk_gemm_select", -1)
         L.call("lsk_gemm_split", 0)
     assert np.array_equal(bits(y), C.w8a8_outlier_linear(x, oidx, wo, W8, ws, bias, "bf16", rot=rot))
+
+
+@pytest.mark.parametrize("M,N,K,ko", [(33, 260, 1024, 16), (300, 516, 1040, 17), (513, 300, 1296, 5), (40, 520, 8192, 9),
+                                      (1025, 2304, 1024, 3)])
+def test_outlier_linear_mid_rows(M, N, K, ko):
+    """The tiles the outlier linear takes by itself past 32 rows: 64-row ones in one round of blocks, a K
+    split of a deep weight, and 128-row ones where 64 rows make two rounds."""
+    from lockstep_amd import lockstep_fullstack as FS
+    say("outlier mid rows", M, N, K, ko)
+    x, oidx, wo, W8, ws, bias = _case(M, N, K, ko, seed=M + N + K + ko)
+    rot = K % 256 == 0
+    y = FS.w8a8_outlier_linear(bf16_dev(x), to_dev(oidx), bf16_dev(wo), to_dev(W8), to_dev(ws), to_dev(bias),
+                               out_dtype=torch.bfloat16, rot=rot)
+    assert np.array_equal(bits(y), C.w8a8_outlier_linear(x, oidx, wo, W8, ws, bias, "bf16", rot=rot))
