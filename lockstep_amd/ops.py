@@ -5,6 +5,7 @@ These are the building blocks of the drop-in modules (`lockstep_fullstack`, `moe
 """
 from __future__ import annotations
 
+from collections import OrderedDict
 
 import torch
 
@@ -309,11 +310,40 @@ def pack_row_pairs(w_nk: torch.Tensor) -> torch.Tensor:
 # exactly as long as the weight, with no cap and no eviction: one more copy of each such weight in HBM
 # (lsk_row_pairs_bytes(N, K), about N * K bytes).  Each entry records the owner's version counter,
 # which every in-place write through the weight or a view of it advances; a stale copy is remade.
+# The pack runs on the stream of the call that makes the copy: any other stream's first use of it waits
+# for the pack's event, and marks the copy as used there, so its memory is not handed out again under
+# that stream's reads.
 # ROW_PAIR_COPIES = False turns the copies off (the GEMMs then read the weights themselves);
 # release_row_pairs(w) frees a weight's copies.  row_pair_packs counts the copies made.
 ROW_PAIR_COPIES = True
 row_pair_packs = 0
 _ATTR = "_lsk_row_pairs"
+
+
+class _RowPairs:
+    """A row-pair copy: the owner's version it was made from, the copy, the event after its pack and the
+    raw handles of the streams ordered after that event."""
+    __slots__ = ("version", "copy", "event", "streams")
+
+    def __init__(self, version, copy):
+        self.version, self.copy, self.event, self.streams = version, copy, None, ()
+        if copy.is_cuda:
+            stream = torch.cuda.current_stream(copy.device)
+            self.event = torch.cuda.Event()
+            self.event.record(stream)
+            self.streams = {stream.cuda_stream}
+
+    def on_current_stream(self):
+        """The copy, readable by later work on the calling thread's current stream."""
+        if self.event is not None and L.stream_of(self.copy) not in self.streams:
+            stream = torch.cuda.current_stream(self.copy.device)
+            stream.wait_event(self.event)
+            self.copy.record_stream(stream)
+            self.streams.add(stream.cuda_stream)
+        return self.copy
+
+    def __reduce__(self):
+        return OrderedDict, ()               # a saved or deep-copied weight goes without: remade on use
 
 
 def _pair_key(w_nk):
@@ -341,13 +371,13 @@ def row_pair_copy(w_nk):
         held = {}
         setattr(owner, _ATTR, held)
     hit = held.get(key)
-    if hit is not None and hit[0] == owner._version:
-        return hit[1]
+    if isinstance(hit, _RowPairs) and hit.version == owner._version:
+        return hit.on_current_stream()
     held.pop(key, None)                      # stale: free it before the new copy is made
-    packed = pack_row_pairs(w_nk)
+    made = _RowPairs(owner._version, pack_row_pairs(w_nk))
     row_pair_packs += 1
-    held[key] = (owner._version, packed)
-    return packed
+    held[key] = made
+    return made.copy
 
 
 def row_pairs_of(w_nk, rows):

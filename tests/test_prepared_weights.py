@@ -144,3 +144,52 @@ def test_copies_can_be_turned_off(counting_pack, monkeypatch):
     monkeypatch.setattr(ops, "ROW_PAIR_COPIES", False)
     assert ops.row_pairs_of(torch.zeros((64, 64), dtype=torch.int8), 4096) is None
     assert counting_pack == []
+
+
+def test_copy_on_another_stream_waits_for_the_pack(monkeypatch):
+    """The copy's pack is ordered on the stream of the call that makes it: another stream's first use
+    waits for the event after it and marks the copy as used there, once; the making stream does neither."""
+    log = []
+
+    class Stream:
+        def __init__(self, handle):
+            self.cuda_stream = handle
+
+        def wait_event(self, event):
+            log.append(("wait", self.cuda_stream, event.at))
+
+    class Event:
+        def record(self, stream):
+            self.at = stream.cuda_stream
+
+    class Copy:
+        is_cuda, device = True, "dev"
+
+        def record_stream(self, stream):
+            log.append(("used", stream.cuda_stream))
+
+    now = [Stream(1)]
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: now[0])
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(L, "stream_of", lambda t: now[0].cuda_stream)
+    copy = Copy()
+    held = ops._RowPairs(0, copy)
+    assert held.on_current_stream() is copy and log == []
+    now[0] = Stream(2)
+    for _ in range(2):
+        assert held.on_current_stream() is copy and log == [("wait", 2, 1), ("used", 2)]
+    now[0] = Stream(1)
+    assert held.on_current_stream() is copy and len(log) == 2
+
+
+def test_weights_with_copies_save_and_deepcopy(counting_pack, tmp_path):
+    """A weight that holds a copy is saved, loaded (weights_only) and deep-copied as before, without the
+    copy, which its own first use makes."""
+    import copy
+    w = torch.arange(64 * 64).view(64, 64).to(torch.int8)
+    first = ops.row_pairs_of(w, 4096)
+    torch.save(w, tmp_path / "w.pt")
+    for t in (torch.load(tmp_path / "w.pt", weights_only=True), copy.deepcopy(w)):
+        assert torch.equal(t, w)
+        assert ops.row_pairs_of(t, 4096) is not first and ops.row_pairs_of(t, 4096) is ops.row_pairs_of(t, 4096)
+    assert ops.row_pairs_of(w, 4096) is first and len(counting_pack) == 3

@@ -67,6 +67,35 @@ def test_captured_dense_linears_follow_in_place_weight_updates():
     assert ops.row_pair_packs == packs + 3
 
 
+def test_copy_read_from_another_stream():
+    """A weight's copy packed behind other work on one stream and read at once from another: both
+    calls' results are the oracle's."""
+    from lockstep_amd import _lib as L
+    from lockstep_amd import lockstep_fullstack as FS
+    g = np.random.default_rng(12)
+    M, N, K = 16, 28672, 256
+    assert L.load().lsk_gemm_reads_row_pairs(M, N, K) == 1
+    x = g.standard_normal((M, K)).astype(np.float32)
+    W8 = g.integers(-127, 128, (N, K), dtype=np.int8)
+    ws = g.uniform(1e-3, 1e-2, N).astype(np.float32)
+    ref = C.w8a8_matmul(x, W8, ws, None, "bf16")
+    xd, sd = to_dev(x), to_dev(ws)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for step in range(2):
+        say("two streams", step)
+        W = to_dev(W8)                                   # a new weight: no copy yet
+        torch.cuda.synchronize()
+        out = []
+        for s in (a, b):
+            with torch.cuda.stream(s):
+                if s is a:
+                    torch.cuda._sleep(20_000_000)        # (clock ticks: the pack waits behind it)
+                out.append(FS.w8a8_matmul(xd, W, sd, out_dtype=torch.bfloat16))
+        torch.cuda.synchronize()
+        for y in out:
+            assert np.array_equal(u16(y), ref), step
+
+
 def test_fifty_expert_lists_pack_once(monkeypatch):
     """50 expert lists (int8 experts, as the reference passes them) through moe_forward at a token
     count whose grouped GEMMs read the experts' row-pair copies, twice, with the table cache bound
