@@ -355,7 +355,8 @@ def row_pair_copy(w_nk):
     """pack_row_pairs(w_nk), made once per weight and kept on the tensor owning its storage while
     that tensor is unchanged; None where the layout does not apply (K % 16 != 0, a strided or
     unaligned weight), while a graph is being captured (the graph then reads the weight itself, so
-    replays follow later in-place updates of it), or with ROW_PAIR_COPIES off."""
+    replays follow later in-place updates of it), for an inference tensor (no version counter tells its
+    updates), or with ROW_PAIR_COPIES off."""
     global row_pair_packs
     if not ROW_PAIR_COPIES or w_nk.dim() != 2 or w_nk.dtype != torch.int8:
         return None
@@ -366,6 +367,8 @@ def row_pair_copy(w_nk):
     if w_nk.is_cuda and torch.cuda.is_current_stream_capturing():
         return None
     owner, key = _pair_key(w_nk)
+    if owner.is_inference():
+        return None
     held = owner.__dict__.get(_ATTR)
     if held is None:
         held = {}

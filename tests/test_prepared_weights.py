@@ -193,3 +193,20 @@ def test_weights_with_copies_save_and_deepcopy(counting_pack, tmp_path):
         assert torch.equal(t, w)
         assert ops.row_pairs_of(t, 4096) is not first and ops.row_pairs_of(t, 4096) is ops.row_pairs_of(t, 4096)
     assert ops.row_pairs_of(w, 4096) is first and len(counting_pack) == 3
+
+
+def test_inference_tensors_go_without_copies(counting_pack):
+    """A weight made under inference mode has no version counter: the GEMMs read it itself, in and out of
+    that mode.  An ordinary weight keeps its copy under inference mode, and in-place writes made there
+    still make it stale."""
+    with torch.inference_mode():
+        w = torch.zeros((64, 64), dtype=torch.int8)
+        assert ops.row_pairs_of(w, 4096) is None
+    assert ops.row_pairs_of(w, 4096) is None and counting_pack == []
+    w = torch.zeros((64, 64), dtype=torch.int8)
+    first = ops.row_pairs_of(w, 4096)
+    with torch.inference_mode():
+        assert ops.row_pairs_of(w.t().t(), 4096) is first
+        w.add_(1)
+        assert ops.row_pairs_of(w, 4096) is not first
+    assert len(counting_pack) == 2
