@@ -246,11 +246,23 @@ def planes_linear(x2: torch.Tensor, w2: torch.Tensor, wbits: int, ws: torch.Tens
     return out
 
 
+def prepare_planes_pairs(w2: torch.Tensor, abits: int):
+    """Make the stacked planes' row-pair copy (kept on w2) where some decode batch reads it (the planes
+    of its activation rows are at most 32 rows)."""
+    pa = 1 if abits == 8 else 2
+    reads = L.load().lsk_gemm_reads_row_pairs
+    if any(reads(n, w2.shape[0], w2.shape[1]) for n in range(pa, 33, pa)):
+        row_pair_copy(w2)
+
+
 def planes_pairs(w2: torch.Tensor, rows: int, abits: int):
-    """The stacked planes' row-pair copy (kept on w2, row_pairs_of) where the planes of `rows`
-    activation rows are a decode batch that reads it (at most 32), else None."""
+    """The copy prepare_planes_pairs made where the planes of `rows` activation rows are a decode batch
+    that reads it, else None: after an in-place update of w2 the planes themselves are read, as no
+    call packs."""
     n = int(rows) * (1 if abits == 8 else 2)
-    return row_pairs_of(w2, n) if n <= 32 and w2.dtype == torch.int8 else None
+    if not 0 < n <= 32 or not L.load().lsk_gemm_reads_row_pairs(n, int(w2.shape[0]), int(w2.shape[1])):
+        return None
+    return row_pair_copy(w2, make=False)
 
 
 def quant8_pow2(x: torch.Tensor, mode: int):
@@ -351,9 +363,9 @@ def _pair_key(w_nk):
     return owner, (w_nk.data_ptr(), int(w_nk.shape[0]), int(w_nk.shape[1]), int(w_nk.stride(0)))
 
 
-def row_pair_copy(w_nk):
+def row_pair_copy(w_nk, make=True):
     """pack_row_pairs(w_nk), made once per weight and kept on the tensor owning its storage while
-    that tensor is unchanged; None where the layout does not apply (K % 16 != 0, a strided or
+    that tensor is unchanged (without `make`: a copy already made, else None); None where the layout does not apply (K % 16 != 0, a strided or
     unaligned weight), while a graph is being captured (the graph then reads the weight itself, so
     replays follow later in-place updates of it), for an inference tensor (no version counter tells its
     updates), or with ROW_PAIR_COPIES off."""
@@ -376,6 +388,8 @@ def row_pair_copy(w_nk):
     hit = held.get(key)
     if isinstance(hit, _RowPairs) and hit.version == owner._version:
         return hit.on_current_stream()
+    if not make:
+        return None
     held.pop(key, None)                      # stale: free it before the new copy is made
     made = _RowPairs(owner._version, pack_row_pairs(w_nk))
     row_pair_packs += 1

@@ -152,21 +152,40 @@ def test_int64_rounding_at_halfway_cases():
     assert np.array_equal(bits(y), f32_bits(want))
 
 
-@pytest.mark.parametrize("spec", ["a15w15", "a8", "w15"])
+@pytest.mark.parametrize("spec,abits,wbits", [("a15w15", 15, 15), ("a8", 8, 8), ("w15", 8, 15)])
 @pytest.mark.parametrize("M,N,K", [(3, 8200, 272), (16, 16385, 64), (17, 8192, 80), (40, 8192, 128)])
-def test_variant_logits_on_row_pairs(spec, M, N, K):
-    """Decode batches of a wide head read the planes' row-pair copy (up to 32 stacked rows; 34 and 80
-    read the planes): the same logits as the planes alone, before and after an in-place update of
-    them, whose copy is remade."""
+def test_variant_logits_on_row_pairs(spec, abits, wbits, M, N, K):
+    """Decode batches of a wide head (5 to 32 rows of stacked planes; 17 rows of two planes are 34) read
+    the row-pair copy that prepare made: the oracle's logits, and no call packs, on the preparing stream
+    and on another, under inference mode, and after an in-place update of the planes, which are then read
+    themselves."""
     from lockstep_amd import ops
     from lockstep_amd import t16h_lmvariants as T
     say("variant pairs", spec, M, N, K)
     r = np.random.default_rng(M + N)
-    W = to_dev((r.standard_normal((N, K)) * 0.05).astype(np.float32))
-    x = to_dev(r.standard_normal((M, K)).astype(np.float32))
-    v = T.build(spec).prepare(W)
-    for step in range(2):
+    W = (r.standard_normal((N, K)) * 0.05).astype(np.float32)
+    xh = r.standard_normal((M, K)).astype(np.float32)
+    reads = 4 < M * (1 if abits == 8 else 2) <= 32
+    x = to_dev(xh)
+    packs = ops.row_pair_packs
+    v = T.build(spec).prepare(to_dev(W))
+    assert ops.row_pair_packs == packs + 1
+    assert (ops.planes_pairs(v._w2, M, abits) is not None) == reads
+    wp, ws = C.quantize_weight_bits(W, wbits)
+    ref = f32_bits(C.mm_planes(xh, wp, ws, abits))
+    assert np.array_equal(bits(v.logits(x)), ref)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
         y = v.logits(x)
-        y0 = ops.planes_linear(x, v._w2, v.wbits, v.ws, v.abits)
-        assert torch.equal(y.view(torch.int32), y0.view(torch.int32)), step
-        v._w2.copy_(v._w2.flip(0).contiguous())
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(y), ref)
+    with torch.inference_mode():
+        assert np.array_equal(bits(v.logits(x)), ref)
+        vi = T.build(spec).prepare(to_dev(W))
+        assert np.array_equal(bits(vi.logits(x)), ref)
+    v._w2.copy_(v._w2.flip(0).contiguous())
+    assert ops.planes_pairs(v._w2, M, abits) is None
+    y0 = ops.planes_linear(x, v._w2, v.wbits, v.ws, v.abits)
+    assert torch.equal(v.logits(x).view(torch.int32), y0.view(torch.int32))
+    assert ops.row_pair_packs == packs + 1

@@ -210,3 +210,22 @@ def test_inference_tensors_go_without_copies(counting_pack):
         w.add_(1)
         assert ops.row_pairs_of(w, 4096) is not first
     assert len(counting_pack) == 2
+
+
+def test_head_planes_pack_in_prepare_only(counting_pack):
+    """A wide head's planes get their copy where prepare asks for it (some decode batch reads it); calls
+    read that copy, or the planes after an in-place update, and never pack.  Narrow heads get none."""
+    w2 = torch.zeros((2 * 8200, 272), dtype=torch.int8)
+    assert ops.planes_pairs(w2, 8, 15) is None and counting_pack == []
+    ops.prepare_planes_pairs(w2, 15)
+    assert len(counting_pack) == 1
+    for rows, abits, reads in ((3, 15, True), (16, 15, True), (17, 15, False), (0, 15, False), (1, 8, False),
+                               (32, 8, True), (33, 8, False)):
+        assert (ops.planes_pairs(w2, rows, abits) is not None) == reads, (rows, abits)
+    w2.add_(1)
+    assert ops.planes_pairs(w2, 8, 15) is None and len(counting_pack) == 1
+    ops.prepare_planes_pairs(w2, 15)
+    assert ops.planes_pairs(w2, 8, 15) is not None and len(counting_pack) == 2
+    for narrow in (torch.zeros((512, 272), dtype=torch.int8), torch.zeros((16400, 40), dtype=torch.int8)):
+        ops.prepare_planes_pairs(narrow, 15)
+    assert len(counting_pack) == 2
