@@ -248,11 +248,14 @@ def planes_linear(x2: torch.Tensor, w2: torch.Tensor, wbits: int, ws: torch.Tens
 
 def prepare_planes_pairs(w2: torch.Tensor, abits: int):
     """Make the stacked planes' row-pair copy (kept on w2) where some decode batch reads it (the planes
-    of its activation rows are at most 32 rows)."""
+    of its activation rows are at most 32 rows) and the device has room for it."""
     pa = 1 if abits == 8 else 2
     reads = L.load().lsk_gemm_reads_row_pairs
     if any(reads(n, w2.shape[0], w2.shape[1]) for n in range(pa, 33, pa)):
-        row_pair_copy(w2)
+        try:
+            row_pair_copy(w2)
+        except torch.OutOfMemoryError:
+            pass                             # the calls read the planes themselves
 
 
 def planes_pairs(w2: torch.Tensor, rows: int, abits: int):

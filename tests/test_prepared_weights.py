@@ -229,3 +229,13 @@ def test_head_planes_pack_in_prepare_only(counting_pack):
     for narrow in (torch.zeros((512, 272), dtype=torch.int8), torch.zeros((16400, 40), dtype=torch.int8)):
         ops.prepare_planes_pairs(narrow, 15)
     assert len(counting_pack) == 2
+
+
+def test_head_planes_without_room_for_the_copy(monkeypatch):
+    """A device with no room for the planes' copy prepares the head without it."""
+    def no_room(w):
+        raise torch.OutOfMemoryError("no room")
+    monkeypatch.setattr(ops, "pack_row_pairs", no_room)
+    w2 = torch.zeros((16400, 64), dtype=torch.int8)
+    ops.prepare_planes_pairs(w2, 15)
+    assert ops.planes_pairs(w2, 8, 15) is None
