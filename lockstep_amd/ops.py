@@ -234,6 +234,7 @@ def planes_linear(x2: torch.Tensor, w2: torch.Tensor, wbits: int, ws: torch.Tens
     if w2.stride(-1) != 1:
         w2 = w2.contiguous()
     N = w2.shape[0] // P
+    _check_pairs(w_pairs, P * N, K, x2.device, "planes_linear")
     out = torch.empty((M, N), dtype=_OUT_T[out_dtype], device=x2.device)
     if M == 0 or N == 0:
         return out
@@ -317,6 +318,12 @@ def pack_row_pairs(w_nk: torch.Tensor) -> torch.Tensor:
     L.call("lsk_pack_row_pairs", L.ptr(w_nk), N, K, w_nk.stride(0) if N > 1 else max(K, 16), L.ptr(out),
            L.stream_of(w_nk))
     return out
+
+
+def _check_pairs(w_pairs, N: int, K: int, device, what: str):
+    if w_pairs is not None and (w_pairs.dtype != torch.int8 or w_pairs.device != device
+                                or w_pairs.numel() < L.load().lsk_row_pairs_bytes(N, K)):
+        raise ValueError("%s: w_pairs is not pack_row_pairs of a [%d, %d] weight" % (what, N, K))
 
 
 # Row-pair copies of weights (the GEMM tiles read them in whole 128-byte lines): a prepared weight,
@@ -443,9 +450,7 @@ def linear_dyn(x: torch.Tensor, w_nk: torch.Tensor, ew: int, stages: int = 3, wo
         work = torch.empty((nbytes + L.load().lsk_gemm_split_bytes(M, N, K),), dtype=torch.uint8, device=x.device)
     elif work.numel() < nbytes:
         raise ValueError("linear_dyn: work buffer of %d bytes, %d needed" % (work.numel(), nbytes))
-    if w_pairs is not None and (w_pairs.dtype != torch.int8 or w_pairs.device != x.device
-                                or w_pairs.numel() < L.load().lsk_row_pairs_bytes(N, K)):
-        raise ValueError("linear_dyn: w_pairs is not pack_row_pairs of a [%d, %d] weight" % (N, K))
+    _check_pairs(w_pairs, N, K, x.device, "linear_dyn")
     L.call("lsk_linear_dyn", L.ptr(x), M, K, x.stride(0) if M > 1 else max(K, 1), L.ptr(w_nk),
            w_nk.stride(0) if N > 1 else max(K, 1), L.ptr(w_pairs), N, int(ew), L.ptr(y),
            y.stride(0) if M > 1 else max(N, 1),

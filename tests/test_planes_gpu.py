@@ -189,3 +189,16 @@ def test_variant_logits_on_row_pairs(spec, abits, wbits, M, N, K):
     y0 = ops.planes_linear(x, v._w2, v.wbits, v.ws, v.abits)
     assert torch.equal(v.logits(x).view(torch.int32), y0.view(torch.int32))
     assert ops.row_pair_packs == packs + 1
+
+
+def test_planes_linear_refuses_foreign_pairs():
+    """w_pairs of another type, device or size than the stacked planes' copy is refused before any launch."""
+    from lockstep_amd import ops
+    x = torch.zeros((8, 64), device=dev())
+    w2 = torch.zeros((2 * 8192, 64), dtype=torch.int8, device=dev())
+    ws = torch.ones((8192,), device=dev())
+    good = ops.pack_row_pairs(w2)
+    for bad in (good[:-1], good.view(torch.uint8), good.cpu()):
+        with pytest.raises(ValueError, match="w_pairs"):
+            ops.planes_linear(x, w2, 15, ws, 15, w_pairs=bad)
+    assert ops.planes_linear(x, w2, 15, ws, 15, w_pairs=good).shape == (8, 8192)
