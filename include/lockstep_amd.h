@@ -669,8 +669,8 @@ int lsk_moe_pp_skinny_rows(int rows);
 /* Tuning control with no counterpart in the reference: the main loop of the grouped MXFP4
  * expert GEMMs (0: direct-to-LDS operand staging with fp4 fragments converted per wave, a
  * two-stage ring, three blocks per CU, the default, and for MXFP4 layers with per-row activation
- * scales past the skinny GEMM the block-scaled MFMA on six-bit activation planes, given exponent
- * bytes in 16 .. 239, mx_safe 0 and act_tab; 1: register-staged operands converted to bf16
+ * scales past the skinny GEMM the block-scaled MFMA on six-bit activation planes, given mx_safe 0
+ * and act_tab; 1: register-staged operands converted to bf16
  * before LDS; 2: as 0 with a three-stage ring and two blocks per CU; 3: as 0, with the skinny
  * grouped MX GEMM -- an expert's rows 16 at a time in LDS, the codes streamed into the bf16 MFMA --
  * wherever the layer can take it, which 0 does by size: MXFP4 layers with per-row activation

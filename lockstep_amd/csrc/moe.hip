@@ -2735,16 +2735,13 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
   const bool pair_w = !mx && moe_reads_pair_weights(T, k, E, H, I, rb) && a->w13_pair_ptrs && a->w2_pair_ptrs;
 
   // MXFP4 experts with per-row scales past the skinny GEMM: six-bit activation planes on the
-  // block-scaled MFMA tiles, for exponent bytes they take (mx6_tile.h).  GPT-OSS-20B on MI355X, bf16
+  // block-scaled MFMA tiles, which take every exponent byte below 240 (mx6_tile.h).  GPT-OSS-20B on MI355X, bf16
   // tiles / these: T = 600 gate/up 293 / 213 us, down 163 / 113; T = 4096 850 / 660 and 380 / 320; the
   // whole layer without skinny copies at T = 32 270 / 189, T = 128 329 / 213, T = 256 389 / 267.  (Against the
   // skinny GEMM, where both can run: T = 32 189 / 135 us, 128 213 / 181, 224 level, 256 266 / 278.)
   const bool use_mx6 = mx == 1 && T > kMxGemvMaxT && !use_mx_skinny && !use_mx_gemv && !a->mx_safe &&
-                       lsk::mx_variant() == 0 &&
-                       std::min(a->kw13_min, a->kw2_min) >= 16 && std::max(a->kw13_max, a->kw2_max) < 240 &&
-                       ((uintptr_t)a->x & 15) == 0 && a->act_tab && ((uintptr_t)a->act_tab & 15) == 0 &&
+                       lsk::mx_variant() == 0 && ((uintptr_t)a->x & 15) == 0 && a->act_tab && ((uintptr_t)a->act_tab & 15) == 0 &&
                        R * H * 2 < 0x7fffffff;
-  const int mx6 = std::max(a->kw13_max, a->kw2_max) <= 180 ? 2 : 1;
   // up to 256 tokens: the dispatch and the row quant of x in one launch
   const bool prep_decode = T <= 256 && rb == 0 && mx != 2 && !use_mx6;
   // routing from logits: inside that launch for up to 4 tokens (a wave per token in its
@@ -2873,7 +2870,7 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
   g1.h_amax = w.h_amax;
   g1.lds = a->lds13;
   if (use_mx6) {
-    g1.mx6 = mx6;
+    g1.mx6 = 1;
     g1.lda = H / 32 * 48;
     g1.a_bytes = T * g1.lda;
   }
@@ -3029,7 +3026,7 @@ static int moe_forward_call(const lsk_moe_args* a, void* stream) {
   g2.y = w.slots;
   g2.lds = a->lds2;
   if (use_mx6) {
-    g2.mx6 = mx6;
+    g2.mx6 = 1;
     g2.y_bytes = R * H * 2;
     g2.lda = I / 32 * 48;
     g2.a_bytes = R * g2.lda;

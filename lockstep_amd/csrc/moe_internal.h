@@ -35,7 +35,7 @@ struct MoeGemmArgs {
   // over tiles without a flagged row; 2 the general kernel over tiles with one
   int mx2;
   // MXFP4 experts, per-row scales: A rows as six-bit planes (lda bytes a row), the block-scaled
-  // MFMA tiles (mx6_tile.h); 2: the E8M0 bytes bound the accumulators (kMx6QuietKexp)
+  // MFMA tiles (mx6_tile.h)
   int mx6;
   int64_t y_bytes;          // bytes of y (mx6)
   const int32_t* row_flag;  // per A row (gate/up: per token)

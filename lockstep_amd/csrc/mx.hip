@@ -553,10 +553,11 @@ __global__ __launch_bounds__(256, RING == 2 ? 3 : 2) void moe_mx_pp_kernel(lsk::
   moe_mx_epilogue<MODE>(a, acc, nt, p0, p1, bias, mx_smem);
 }
 
-// Whether no output of a row with scale asc, routing weight w and column bias b can be NaN, given
-// the accumulators' bound of 2^81 (E8M0 bytes up to kMx6QuietKexp and K < 2^18: 2^13 blocks of 2^15
-// 2^53): finite scales and biases keep every product and sum finite.
-constexpr int kMx6QuietKexp = 180;
+// No output of a row with scale asc < 2^40, routing weight w < 2^40 and column bias b < 2^96 can be
+// NaN where the accumulators are below 2^81: every product and sum of them stays finite.  The wave
+// looks at its own accumulators (a bound taken from the weights' E8M0 bytes on the host would go stale
+// when a program writes new ones in place); none is NaN, as every block's sum is finite.
+constexpr float kMx6Quiet = 0x1p81f;
 
 // Two binary32 values rounded to bf16, packed; QUIET: neither is NaN.
 template <bool QUIET>
@@ -734,7 +735,14 @@ __global__ __launch_bounds__(256, 2) void moe_mx6_kernel(lsk::MoeGemmArgs a) {
   if (na == 0) return;
   const __amdgpu_buffer_rsrc_t ro = MODE == 0 ? lsk::make_rsrc(a.h + (int64_t)p0 * a.N, (int64_t)(p1 - p0) * a.N * 2)
                                               : lsk::make_rsrc(a.y, a.y_bytes);
-  bool qb = a.mx6 == 2 && quiet;
+  float top = 0.0f;
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) top = fmaxf(top, fabsf(acc[i][j][r]));
+  bool qb = quiet && __builtin_amdgcn_ballot_w64(!(top < kMx6Quiet)) == 0;
   if (bias) {
     const int col = MODE == 0 ? nt * 64 + wn * 32 + (lane & 31) : nt * 128 + wn * 64 + lane;
     const bool ok = col >= a.N || (fabsf(bias[col]) < 0x1p96f && (MODE == 1 || fabsf(bias[a.N + col]) < 0x1p96f));

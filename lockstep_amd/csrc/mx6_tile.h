@@ -11,15 +11,15 @@
 // same 16 bytes of packed E2M1 codes as they lie in memory, under the weight's own E8M0 byte.  From
 // a zero accumulator the result is s_b * 2^(kexp - 128) exactly: the products are multiples of
 // 2^(kexp - 128) and sum to less than 2^16 of them (checked against binary64 on MI355X over 20 M
-// sums with kexp 1 .. 239; the accumulator input is not rounded once, so the update stays on the
+// sums with kexp 0 .. 239, 3 M of them at each of 0 .. 19; the accumulator input is not rounded once, so the update stays on the
 // VALU).  The update is then one binary32 add per output and block, with no scale to read, no fp4
 // conversions and half the matrix-core time of the bf16 form (16 adds of 4 cycles against one MFMA
 // of 32 cycles per 32 x 32 outputs and block; bf16: 64).  The adds bound the loop, so the rest of
 // it is kept off the VALU: all operands go global -> LDS by direct buffer loads with exact counted
 // waits, and a wave whose rows are empty (experts fill few of a tile's 128 rows) skips its strips.
 //
-// Exponent bytes of 240 and more could overflow the product and those under 16 come near the
-// subnormals, so other weight sets take the bf16 tiles (mx_pp.h).
+// Exponent bytes of 240 and more could overflow the product, so weight sets that hold one (the
+// layer's mx_safe) take the bf16 tiles (mx_pp.h); the sums of the smallest are subnormal and exact.
 //
 // A rows: 48 bytes per block -- [high 0..15][high 16..23, low 16..23][low 0..15], code i of a
 // plane at bits 6 i .. 6 i + 5 -- written by the row quantisers (mx.hip).  A lane's six registers
@@ -35,8 +35,6 @@ namespace lsk {
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-
-constexpr int kMx6KexpMin = 16;  // E8M0 bytes the six-bit form takes (to 239)
 
 struct Mx6Cfg {
   static constexpr int BM = 128, BN = 128, kThreads = 256;
