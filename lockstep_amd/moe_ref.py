@@ -225,7 +225,7 @@ class ExpertTables:
         self.b2 = table(b2) if any(b2) else None
         # the weights' row-pair copies, which the ping-pong expert tiles read in whole 128-byte
         # lines (the decode GEMVs and the other tiles read the weights above): made by pair_ptrs()
-        # on the first call that reads them, held by each weight tensor (ops.row_pair_copy)
+        # on the first call that reads them, held by each weight tensor (ops.row_pair_copies)
         self.w13_pairs = self.w2_pairs = None
         self._w13, self._w2 = w13, w2
         self._keep = keep
@@ -247,12 +247,12 @@ class ExpertTables:
         if not ROW_PAIRS or self.H % 16 or self.I % 16:
             return None, None
         if self.w13_pairs is None:
-            p13 = [ops.row_pair_copy(t) for t in self._w13]
-            p2 = [ops.row_pair_copy(t) for t in self._w2]
-            if any(t is None for t in p13 + p2):
+            copies = ops.row_pair_copies(self._w13 + self._w2)
+            if any(t is None for t in copies):
                 return None, None              # (being captured into a graph: the weights themselves)
             dev = self.device
-            self._pairs_keep = p13 + p2
+            p13, p2 = copies[:self.E], copies[self.E:]
+            self._pairs_keep = copies
             self.w13_pairs = torch.tensor([t.data_ptr() for t in p13], dtype=torch.int64).to(dev)
             self.w2_pairs = torch.tensor([t.data_ptr() for t in p2], dtype=torch.int64).to(dev)
         return self.w13_pairs, self.w2_pairs
@@ -267,7 +267,7 @@ def _derived(pairs):
 # Tables of the experts lists the layers have seen, keyed by the list and its per-expert tuples.  A
 # table holds device address tables (a few KB) and references to the list's tensors; the large
 # derived data, the int8 weights' row-pair copies, is held by the weight tensors themselves
-# (ops.row_pair_copy), so a table rebuilt after eviction re-packs nothing.  TABLES_MAX bounds how
+# (ops.row_pair_copies), so a table rebuilt after eviction re-packs nothing.  TABLES_MAX bounds how
 # many lists keep their tensors referenced here (more than the MoE layers of the largest model
 # served: Qwen3-30B-A3B has 48).
 _TABLES = {}

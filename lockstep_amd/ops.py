@@ -344,16 +344,11 @@ _ATTR = "_lsk_row_pairs"
 
 class _RowPairs:
     """A row-pair copy: the owner's version it was made from, the copy, the event after its pack and the
-    raw handles of the streams ordered after that event."""
+    raw handles of the streams ordered after that event (none off the GPU)."""
     __slots__ = ("version", "copy", "event", "streams")
 
     def __init__(self, version, copy):
         self.version, self.copy, self.event, self.streams = version, copy, None, ()
-        if copy.is_cuda:
-            stream = torch.cuda.current_stream(copy.device)
-            self.event = torch.cuda.Event()
-            self.event.record(stream)
-            self.streams = {stream.cuda_stream}
 
     def on_current_stream(self):
         """The copy, readable by later work on the calling thread's current stream."""
@@ -368,43 +363,64 @@ class _RowPairs:
         return OrderedDict, ()               # a saved or deep-copied weight goes without: remade on use
 
 
+def _packed_on_current_stream(made):
+    """One event behind the packs of new copies on one device."""
+    if made and made[0].copy.is_cuda:
+        stream = torch.cuda.current_stream(made[0].copy.device)
+        event = torch.cuda.Event()
+        event.record(stream)
+        for m in made:
+            m.event, m.streams = event, {stream.cuda_stream}
+
+
 def _pair_key(w_nk):
     owner = w_nk._base if w_nk._base is not None else w_nk
     return owner, (w_nk.data_ptr(), int(w_nk.shape[0]), int(w_nk.shape[1]), int(w_nk.stride(0)))
 
 
-def row_pair_copy(w_nk, make=True):
-    """pack_row_pairs(w_nk), made once per weight and kept on the tensor owning its storage while
-    that tensor is unchanged (without `make`: a copy already made, else None); None where the layout does not apply (K % 16 != 0, a strided or
-    unaligned weight), while a graph is being captured (the graph then reads the weight itself, so
-    replays follow later in-place updates of it), for an inference tensor (no version counter tells its
-    updates), or with ROW_PAIR_COPIES off."""
+def row_pair_copies(weights, make=True):
+    """Per weight of one device: pack_row_pairs(w_nk), made once per weight and kept on the tensor owning
+    its storage while that tensor is unchanged (without `make`: a copy already made, else None); None
+    where the layout does not apply (K % 16 != 0, a strided or unaligned weight), while a graph is being
+    captured (the graph then reads the weight itself, so replays follow later in-place updates of it),
+    for an inference tensor (no version counter tells its updates), or with ROW_PAIR_COPIES off."""
     global row_pair_packs
-    if not ROW_PAIR_COPIES or w_nk.dim() != 2 or w_nk.dtype != torch.int8:
-        return None
-    N, K = w_nk.shape
-    if K == 0 or N == 0 or K % 16 != 0 or w_nk.stride(1) != 1 or w_nk.stride(0) % 16 != 0 \
-            or w_nk.data_ptr() % 16 != 0:
-        return None
-    if w_nk.is_cuda and torch.cuda.is_current_stream_capturing():
-        return None
-    owner, key = _pair_key(w_nk)
-    if owner.is_inference():
-        return None
-    held = owner.__dict__.get(_ATTR)
-    if held is None:
-        held = {}
-        setattr(owner, _ATTR, held)
-    hit = held.get(key)
-    if isinstance(hit, _RowPairs) and hit.version == owner._version:
-        return hit.on_current_stream()
-    if not make:
-        return None
-    held.pop(key, None)                      # stale: free it before the new copy is made
-    made = _RowPairs(owner._version, pack_row_pairs(w_nk))
-    row_pair_packs += 1
-    held[key] = made
-    return made.copy
+    out, made = [], []
+    for w_nk in weights:
+        out.append(None)
+        if not ROW_PAIR_COPIES or w_nk.dim() != 2 or w_nk.dtype != torch.int8:
+            continue
+        N, K = w_nk.shape
+        if K == 0 or N == 0 or K % 16 != 0 or w_nk.stride(1) != 1 or w_nk.stride(0) % 16 != 0 \
+                or w_nk.data_ptr() % 16 != 0:
+            continue
+        if w_nk.is_cuda and torch.cuda.is_current_stream_capturing():
+            continue
+        owner, key = _pair_key(w_nk)
+        if owner.is_inference():
+            continue
+        held = owner.__dict__.get(_ATTR)
+        if held is None:
+            held = {}
+            setattr(owner, _ATTR, held)
+        hit = held.get(key)
+        if isinstance(hit, _RowPairs) and hit.version == owner._version:
+            out[-1] = hit.on_current_stream()
+        elif make:
+            held.pop(key, None)              # stale: free it before the new copy is made
+            new = _RowPairs(owner._version, pack_row_pairs(w_nk))
+            row_pair_packs += 1
+            made.append((held, key, new))
+            out[-1] = new.copy
+    _packed_on_current_stream([m for _, _, m in made])
+    for held, key, new in made:              # (stored once the event is behind their packs)
+        held[key] = new
+    return out
+
+
+def row_pair_copy(w_nk, make=True):
+    """row_pair_copies of one weight."""
+    return row_pair_copies([w_nk], make)[0]
 
 
 def row_pairs_of(w_nk, rows):

@@ -174,12 +174,25 @@ def test_copy_on_another_stream_waits_for_the_pack(monkeypatch):
     monkeypatch.setattr(L, "stream_of", lambda t: now[0].cuda_stream)
     copy = Copy()
     held = ops._RowPairs(0, copy)
+    ops._packed_on_current_stream([held])
     assert held.on_current_stream() is copy and log == []
     now[0] = Stream(2)
     for _ in range(2):
         assert held.on_current_stream() is copy and log == [("wait", 2, 1), ("used", 2)]
     now[0] = Stream(1)
     assert held.on_current_stream() is copy and len(log) == 2
+
+
+def test_an_expert_list_shares_one_event(counting_pack, monkeypatch):
+    """The copies of a list of weights are stored with one event, recorded once behind all their packs."""
+    calls = []
+    monkeypatch.setattr(ops, "_packed_on_current_stream", lambda made: calls.append((len(counting_pack), len(made))))
+    ws = [torch.zeros((64, 64), dtype=torch.int8) for _ in range(5)]
+    copies = ops.row_pair_copies(ws)
+    assert calls == [(5, 5)] and all(c is ops.row_pairs_of(w, 4096) for c, w in zip(copies, ws))
+    ws[2].add_(1)
+    again = ops.row_pair_copies(ws)
+    assert [a is c for a, c in zip(again, copies)] == [True, True, False, True, True] and (6, 1) in calls
 
 
 def test_weights_with_copies_save_and_deepcopy(counting_pack, tmp_path):
