@@ -284,8 +284,8 @@ int lsk_quant8_dyn_single_pass(int on);
 /* Tuning control with no counterpart in the reference: the quantise pass of lsk_linear_dyn's
  * quant8_dyn (0: row pairs per block; 1, the default: a contiguous tensor with K % 64 == 0 and M
  * even walked in the order of q, a wave's stores covering two whole 128-byte lines of q, 0
- * otherwise; from 64 MB of x the exponent guessed from every 32nd row and the pass repeated only if
- * the whole maximum says otherwise; 2: as 1 without the guess and with ordinary rather than
+ * otherwise; from 64 MB of x the exponent guessed from a 32nd of it and only what a wrong guess
+ * quantised repeated; 2: as 1 without the guess and with ordinary rather than
  * non-temporal loads in both passes).  The same exponent and q.  Thread-local. */
 int lsk_quant8_dyn_variant(int v);
 

@@ -268,72 +268,73 @@ LSK_DEV uint32_t quant_pow2_x4(float4 v, float sc) {
          ((uint32_t)(uint8_t)quant_pow2_one(v.z, sc) << 16) | ((uint32_t)(uint8_t)quant_pow2_one(v.w, sc) << 24);
 }
 
-// The quantise passes' STAGE 0 derives the exponent from every block's maximum.  A contiguous tensor
-// of kSpecBytes and more is quantised on a guessed exponent instead, so
-// that x is read once where the guess holds (dyn_sample_kernel takes the maximum of 1 row in 32, and
-// the guess allows for a whole maximum 9% above it): STAGE 1 derives the exponent from the sample's
-// maxima, quantises, and leaves its run's own maximum in own[blockIdx.x] and the exponent in *guess;
-// STAGE 2 reduces those maxima, writes the tensor's exponent and returns, or, where the guess was
-// another, quantises again.  (MI355X, us, 8192 x 18944 binary32: maxima + quantise 97 + 138; sample + STAGE
-// 1 + 2 with the guess right 154, wrong 289.  On N(0,1) the maximum of 1 row in 32 is about 0.88 of
-// the whole, so with the headroom few scales guess wrong.)
-constexpr int64_t kSpecBytes = 64 << 20;  // (69 MB: 34 us as two passes, 24 guessed, 39 guessed wrong; not measured below)
+// A contiguous tensor of kSpecBytes and more is quantised on a guessed exponent, so that x is read once
+// where the guess holds.  dyn_sample_kernel takes the maximum of one 256-byte piece in 32, at a place
+// that varies from group to group (so every column is seen in some rows, and every long row in part),
+// and of the whole first row, where activations have their largest values.  Where most partial maxima
+// of the sample are within a factor of two of its maximum, the guess allows for a whole maximum 9% above it
+// (on N(0,1) the sample's is about 0.88 of the whole's); a sample of a few far larger values likely
+// holds the largest, and headroom that crosses a power of two which the maximum does not costs the whole
+// second pass.  How a wrong guess is put right stands at dyn_quant_pair_flat_kernel.
+constexpr int64_t kSpecBytes = 64 << 20;
 constexpr int kSpecSamples = 512;
 constexpr float kSpecHeadroom = 1.09f;
 
-// The maximum of rows 0, 32, 64, ... (whole rows: every column, and the first row, where activations
-// have their largest values), kSpecSamples partial maxima.
+// Behind the kDynBlocks partial maxima in linear_dyn's workspace.
+struct SpecWords {
+  float sample[kSpecSamples];   // the sample's maxima
+  int32_t cur;                  // the least exponent that a value seen so far allows
+  int32_t rec[kDynBlocks * 4];  // per wave: its last exponent + 32, and the first step under it times 128
+};
+
+// The largest magnitude that exponent e represents: pow2_exponent(m) >= e up to it.
+LSK_DEV float spec_limit(int e) { return e <= -32 ? __builtin_inff() : f32_mul(127.0f, pow2f(-e)); }
+
 __global__ __launch_bounds__(256) void dyn_sample_kernel(const float* __restrict__ x, int64_t M, int64_t K,
-                                                         float* __restrict__ out) {
+                                                         SpecWords* __restrict__ w) {
   __shared__ float red[4];
-  const int k4 = (int)(K >> 2);
-  const int64_t n = (M + 31) / 32 * k4;
+  constexpr int kPiece = 16, kGroup = 32 * kPiece;  // float4s
+  const float4* x4 = (const float4*)x;
+  const int n4 = (int)((M * K) >> 2);
+  const int n = (n4 + kGroup - 1) / kGroup * kPiece;
   float am = 0.0f;
   constexpr int U = 4;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)kSpecSamples * 256 * U) {
+  for (int i = (int)blockIdx.x * 256 + (int)threadIdx.x; i < n; i += kSpecSamples * 256 * U) {
     float4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t j = i + (int64_t)u * kSpecSamples * 256;
-      const int64_t f = j < n ? j : i;
-      const int64_t r = f / k4;
-      v[u] = ((const float4*)(x + r * 32 * K))[f - r * k4];
+      const int t = i + u * kSpecSamples * 256;
+      const uint32_t g = (uint32_t)t / kPiece;
+      const int64_t f = (int64_t)g * kGroup + ((g * 0x9E3779B1u) >> 27) * kPiece + (uint32_t)t % kPiece;
+      v[u] = x4[f < n4 ? f : 0];
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
       am = fmaxf(am, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
   }
+  for (int i = (int)blockIdx.x * 256 + (int)threadIdx.x; i < (int)(K >> 2); i += kSpecSamples * 256) {
+    const float4 v = x4[i];
+    am = fmaxf(am, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+  }
   am = block_max<256>(am, red);
-  if (threadIdx.x == 0) out[blockIdx.x] = am;
+  if (threadIdx.x == 0) w->sample[blockIdx.x] = am;
+  if (blockIdx.x == 0 && threadIdx.x == 0) w->cur = INT32_MAX;
 }
 
-template <int STAGE = 0>
 __global__ __launch_bounds__(256) void dyn_quant_kernel(const float* __restrict__ x, int64_t M, int64_t K,
                                                         int64_t ldx, int flat, const float* __restrict__ partial,
                                                         int nparts, int8_t* __restrict__ q, int64_t ldq,
-                                                        int32_t* __restrict__ e_out, int32_t* __restrict__ erow,
-                                                        float* __restrict__ own, int32_t* __restrict__ guess) {
+                                                        int32_t* __restrict__ e_out, int32_t* __restrict__ erow) {
   __shared__ float red[4];
   float am = 0.0f;
   for (int j = threadIdx.x; j < nparts; j += 256) am = fmaxf(am, partial[j]);
   am = block_max<256>(am, red);
-  // 0 for an all-zero tensor, whose q is then 0 as well
-  const int e = pow2_exponent(STAGE == 1 ? f32_mul(am, kSpecHeadroom) : am);
+  const int e = pow2_exponent(am);   // 0 for an all-zero tensor, whose q is then 0 as well
   const float sc = pow2f(e);         // e in [-32, 40]: a normal power of two
   const int64_t stride = (int64_t)gridDim.x * 256;
-  if constexpr (STAGE == 1) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *guess = e;
-  } else {
-    if (blockIdx.x == 0 && threadIdx.x == 0) e_out[0] = e;
-    if (erow)
-      for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < M; r += stride) erow[r] = e;
-  }
-  if (STAGE == 2 && *guess == e) return;
-  float mine = 0.0f;
-  auto see = [&](const float4& v) {
-    if constexpr (STAGE == 1)
-      mine = fmaxf(mine, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-  };
+  if (blockIdx.x == 0 && threadIdx.x == 0) e_out[0] = e;
+  if (erow)
+    for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < M; r += stride) erow[r] = e;
   if (flat) {
     // pairs of float4 (eight elements, one 8-byte store of q), each block a contiguous run
     const int64_t n8 = (M * K) >> 3;
@@ -350,27 +351,15 @@ __global__ __launch_bounds__(256) void dyn_quant_kernel(const float* __restrict_
         v[u][1] = ld_nt(x4 + 2 * (i + 256 * u) + 1);
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        see(v[u][0]);
-        see(v[u][1]);
+      for (int u = 0; u < U; ++u)
         *(v2u32*)(q + 8 * (i + 256 * u)) = v2u32{quant_pow2_x4(v[u][0], sc), quant_pow2_x4(v[u][1], sc)};
-      }
     }
     for (; i < b1; i += 256) {
       const float4 a = ld_nt(x4 + 2 * i), b = ld_nt(x4 + 2 * i + 1);
-      see(a);
-      see(b);
       *(v2u32*)(q + 8 * i) = v2u32{quant_pow2_x4(a, sc), quant_pow2_x4(b, sc)};
     }
     if (blockIdx.x == gridDim.x - 1)
-      for (int64_t j = (n8 << 3) + threadIdx.x; j < M * K; j += 256) {
-        if (STAGE == 1) mine = fmaxf(mine, fabsf(x[j]));
-        q[j] = quant_pow2_one(x[j], sc);
-      }
-    if constexpr (STAGE == 1) {
-      mine = block_max<256>(mine, red);
-      if (threadIdx.x == 0) own[blockIdx.x] = mine;
-    }
+      for (int64_t j = (n8 << 3) + threadIdx.x; j < M * K; j += 256) q[j] = quant_pow2_one(x[j], sc);
   } else {
     for (int64_t r = blockIdx.x; r < M; r += gridDim.x)
       for (int64_t c = threadIdx.x; c < K; c += 256) q[r * ldq + c] = quant_pow2_one(x[r * ldx + c], sc);
@@ -454,13 +443,27 @@ __global__ __launch_bounds__(256) void dyn_quant_pair_kernel(const float* __rest
 // rows of a pair) and its load four 256-byte runs of x (a chunk of each row of the pair, twice).
 // Every load of a step is issued before any is used, none under a branch (a lane past the run
 // re-reads the run's first float4 and stores nothing).
+//
+// STAGE 0: partial holds the blocks' maxima of dyn_amax_kernel.  On a guessed exponent: STAGE 1 starts
+// each wave on the sample's exponent and lowers it where a value needs that, telling the other
+// waves through w->cur, which each looks at once a step; a wave leaves its last exponent and the step
+// it came into force at in w->rec, and the block its run's maximum in own.  STAGE 2 reduces those
+// maxima, writes the tensor's exponent and quantises again the steps that a wave ran under another
+// one.  So a value that proves the guess wrong costs the steps before it was met, not the whole pass.
+// PAIR: q in the row-pair layout, else as x lies (unit f is float4 f).
+// MI355X, us, against maxima + quantise, means over 8 tensors (2 for the first and last): 620 MB (231 as
+// two passes) N(0,1) 149, silu(g) u of normals 182, Student's t of 5 degrees 176, lognormal row scales
+// 192, one row of massive values 196, eight 152, the largest value last 284; 117 MB (47.5, the second read
+// from the last-level cache) 36, 43, 49, 37, 50, 40, 60; 68 MB (37) 28, 28, 32, 34, 37, 32, 43.  (With
+// the whole pass repeated after any wrong guess: 620 MB 155, 222, 273, 255, 289, 272, 289.)
 constexpr int kDynU2 = 8;
-template <bool NT, int STAGE = 0>
+
+template <bool NT, int STAGE = 0, bool PAIR = true>
 __global__ __launch_bounds__(256) void dyn_quant_pair_flat_kernel(const float* __restrict__ x, int64_t M, int64_t K,
                                                                   const float* __restrict__ partial, int nparts,
                                                                   int8_t* __restrict__ q, int32_t* __restrict__ e_out,
                                                                   int32_t* __restrict__ erow,
-                                                                  float* __restrict__ own, int32_t* __restrict__ guess) {
+                                                                  float* __restrict__ own, SpecWords* __restrict__ w) {
   __shared__ float red[4];
   const int n4 = (int)((M * K) >> 2);
   const int per = (n4 + (int)gridDim.x - 1) / (int)gridDim.x;
@@ -469,12 +472,12 @@ __global__ __launch_bounds__(256) void dyn_quant_pair_flat_kernel(const float* _
   const int K2 = 2 * (int)K;
   // q byte 4 f as (row pair pp, offset rem in the pair's 2K bytes); each step of 256 units adds 1024
   const int f0 = b0 + (int)threadIdx.x;
-  int pp = (4 * f0) / K2, rem = 4 * f0 - pp * K2;
-  const int dp = 1024 / K2, drem = 1024 - dp * K2;
+  int pp = PAIR ? (4 * f0) / K2 : 0, rem = PAIR ? 4 * f0 - pp * K2 : 0;
+  const int dp = PAIR ? 1024 / K2 : 0, drem = PAIR ? 1024 - dp * K2 : 0;
   auto src = [&](int f, int p, int r) {
     // element (2p + (r >> 6 & 1), 64 (r >> 7) + (r & 63)) of x, as a float4 index
     const int e = (2 * p + ((r >> 6) & 1)) * (int)K + 64 * (r >> 7) + (r & 63);
-    return x4 + (f < b1 ? (e >> 2) : b0);
+    return x4 + (f < b1 ? (PAIR ? e >> 2 : f) : b0);
   };
   auto load = [&](const float4* p) {
     if constexpr (NT) return ld_nt(p);
@@ -486,6 +489,7 @@ __global__ __launch_bounds__(256) void dyn_quant_pair_flat_kernel(const float* _
     for (int u = 0; u < kDynU2; ++u) {
       lp[u] = pp;
       lr[u] = rem;
+      if constexpr (!PAIR) continue;
       pp += dp;
       rem += drem;
       if (rem >= K2) {
@@ -497,52 +501,95 @@ __global__ __launch_bounds__(256) void dyn_quant_pair_flat_kernel(const float* _
   // the first step requested before the partial maxima are reduced (it does not depend on them)
   float4 v[kDynU2];
   int f = f0;
-  auto first = [&]() {
+  auto fetch = [&]() {
     addrs();
 #pragma unroll
     for (int u = 0; u < kDynU2; ++u) v[u] = load(src(f + 256 * u, lp[u], lr[u]));
   };
-  if (STAGE != 2 && b0 < b1) first();
+  if (STAGE != 2 && b0 < b1) fetch();
   float am = 0.0f;
   for (int j = threadIdx.x; j < nparts; j += 256) am = fmaxf(am, partial[j]);
+  const float part = am;
   am = block_max<256>(am, red);
-  const int e = pow2_exponent(STAGE == 1 ? f32_mul(am, kSpecHeadroom) : am);
-  const float sc = pow2f(e);
-  if constexpr (STAGE == 1) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *guess = e;
-  } else {
+  int e = pow2_exponent(STAGE == 1 && __syncthreads_count(part > 0.5f * am) >= 128 ? f32_mul(am, kSpecHeadroom) : am);
+  float sc = pow2f(e);
+  if constexpr (STAGE != 1) {
     if (blockIdx.x == 0 && threadIdx.x == 0) e_out[0] = e;
     if (erow)
       for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < M; r += (int64_t)gridDim.x * 256) erow[r] = e;
   }
-  if constexpr (STAGE == 2) {
-    if (*guess == e) return;
-    if (b0 < b1) first();
-  }
-  float mine = 0.0f;
-  auto run_max = [&]() {
-    if constexpr (STAGE == 1) {
-#pragma unroll
-      for (int u = 0; u < kDynU2; ++u)
-        mine = fmaxf(mine, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
-    }
-  };
   uint32_t* q4 = (uint32_t*)q;
-  for (; f < b1;) {
-    run_max();  // (a lane past the run holds the run's first float4)
+  auto store = [&]() {
 #pragma unroll
     for (int u = 0; u < kDynU2; ++u)
       if (f + 256 * u < b1) q4[f + 256 * u] = quant_pow2_x4(v[u], sc);
     f += 256 * kDynU2;
-    if (f >= b1) break;
-    addrs();
-#pragma unroll
-    for (int u = 0; u < kDynU2; ++u) v[u] = load(src(f + 256 * u, lp[u], lr[u]));
+  };
+  if constexpr (STAGE == 0) {
+    if (b0 >= b1) return;
+    for (;;) {
+      store();
+      if (f >= b1) break;
+      fetch();
+    }
+    return;
   }
+  // (from here on by whole waves: lanes past the run hold its first float4)
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int steps = (b1 - b0 - wave * 64 + 256 * kDynU2 - 1) / (256 * kDynU2);  // (<= 0: no units)
   if constexpr (STAGE == 1) {
+    float mine = 0.0f;
+    int since = 0;
+    auto poll = [&]() { return __hip_atomic_load(&w->cur, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    int cur = poll();
+    for (int s = 0; s < steps; ++s) {
+      float m = 0.0f;
+#pragma unroll
+      for (int u = 0; u < kDynU2; ++u)
+        m = fmaxf(m, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
+      mine = fmaxf(mine, m);
+      int now = min(e, __builtin_amdgcn_readfirstlane(cur));
+      if (__builtin_amdgcn_ballot_w64(m > spec_limit(now))) {
+        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+        now = __builtin_amdgcn_readfirstlane(pow2_exponent(m));
+        if (lane == 0) atomicMin(&w->cur, now);
+      }
+      if (now != e) {
+        e = now;
+        sc = pow2f(e);
+        since = s;
+      }
+      store();
+      if (s + 1 < steps) {
+        cur = poll();
+        fetch();
+      }
+    }
+    if (lane == 0) w->rec[blockIdx.x * 4 + wave] = since * 128 + e + 32;
     mine = block_max<256>(mine, red);
     if (threadIdx.x == 0) own[blockIdx.x] = mine;
+  } else {
+    const int rec = w->rec[blockIdx.x * 4 + wave];
+    const int redo = (rec & 127) - 32 == e ? rec >> 7 : steps;
+    for (int s = 0; s < redo; ++s) {
+      fetch();
+      store();
+    }
   }
+}
+
+// The launches of the guessed exponent (x contiguous and 16-byte aligned, K % 4 == 0, M K < 2^31, q 4-byte
+// aligned; PAIR: K % 64 == 0 and M even too).
+template <bool PAIR>
+int launch_spec(const float* x, int64_t M, int64_t K, int8_t* q, int32_t* e_out, int32_t* erow, float* partial,
+                hipStream_t s) {
+  SpecWords* w = (SpecWords*)(partial + kDynBlocks);
+  hipLaunchKernelGGL(dyn_sample_kernel, dim3(kSpecSamples), dim3(256), 0, s, x, M, K, w);
+  hipLaunchKernelGGL((dyn_quant_pair_flat_kernel<true, 1, PAIR>), dim3(kDynBlocks), dim3(256), 0, s, x, M, K,
+                     (const float*)w->sample, kSpecSamples, q, e_out, erow, partial, w);
+  hipLaunchKernelGGL((dyn_quant_pair_flat_kernel<true, 2, PAIR>), dim3(kDynBlocks), dim3(256), 0, s, x, M, K,
+                     (const float*)partial, kDynBlocks, q, e_out, erow, (float*)nullptr, w);
+  return lsk::check_launch("dyn_quant_pair_flat_kernel");
 }
 
 // Single-pass quant8_dyn into the row-pair layout for a tensor that fits on chip (a cooperative
@@ -652,29 +699,21 @@ __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* __restrict__ p,
 }
 
 // Launches of quant8_dyn on a workspace of kDynBlocks floats.
-// spec: partial has room for the sample's maxima and the guess behind the blocks' maxima (linear_dyn's
-// workspace), so a large contiguous tensor is quantised on a guessed exponent.
+// spec: partial has room for SpecWords behind the blocks' maxima (linear_dyn's workspace), so a large
+// contiguous tensor is quantised on a guessed exponent.
 int launch_quant8_dyn(const float* x, int64_t M, int64_t K, int64_t ldx, int8_t* q, int64_t ldq, int32_t* e_out,
                       int32_t* erow, float* partial, bool spec, hipStream_t s) {
   const int64_t total = M * K;
   const int flat = (ldx == K && ldq == K && ((uintptr_t)x % 16) == 0 && ((uintptr_t)q % 8) == 0) ? 1 : 0;
   int64_t blocks = flat ? (total + 256 * 16 - 1) / (256 * 16) : M;
   blocks = blocks < 1 ? 1 : (blocks > kDynBlocks ? kDynBlocks : blocks);
-  if (spec && flat && K % 4 == 0 && 4 * total >= kSpecBytes) {
-    float* sample = partial + kDynBlocks;
-    int32_t* guess = (int32_t*)(sample + kSpecSamples);
-    hipLaunchKernelGGL(dyn_sample_kernel, dim3(kSpecSamples), dim3(256), 0, s, x, M, K, sample);
-    hipLaunchKernelGGL(dyn_quant_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat,
-                       (const float*)sample, kSpecSamples, q, ldq, e_out, erow, partial, guess);
-    hipLaunchKernelGGL(dyn_quant_kernel<2>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat,
-                       (const float*)partial, (int)blocks, q, ldq, e_out, erow, (float*)nullptr, guess);
-    return lsk::check_launch("dyn_quant_kernel");
-  }
+  if (spec && flat && K % 4 == 0 && 4 * total >= kSpecBytes && total < (int64_t)1 << 31)
+    return launch_spec<false>(x, M, K, q, e_out, erow, partial, s);
   hipLaunchKernelGGL(dyn_amax_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat, partial);
   int rc = lsk::check_launch("dyn_amax_kernel");
   if (rc) return rc;
-  hipLaunchKernelGGL(dyn_quant_kernel<0>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat,
-                     (const float*)partial, (int)blocks, q, ldq, e_out, erow, (float*)nullptr, (int32_t*)nullptr);
+  hipLaunchKernelGGL(dyn_quant_kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat,
+                     (const float*)partial, (int)blocks, q, ldq, e_out, erow);
   return lsk::check_launch("dyn_quant_kernel");
 }
 
@@ -739,16 +778,8 @@ int launch_quant8_dyn_pair(const float* x, int64_t M, int64_t K, int64_t ldx, in
                         ((uintptr_t)q % 4) == 0;
   int64_t fb = (total / 4 + 256 * kDynU2 * 2 - 1) / (256 * kDynU2 * 2);
   fb = fb < 1 ? 1 : (fb > kDynBlocks ? kDynBlocks : fb);
-  if (in_order && g_dynq == 1 && 4 * total >= kSpecBytes) {
-    float* sample = partial + kDynBlocks;
-    int32_t* guess = (int32_t*)(sample + kSpecSamples);
-    hipLaunchKernelGGL(dyn_sample_kernel, dim3(kSpecSamples), dim3(256), 0, s, x, M, K, sample);
-    hipLaunchKernelGGL((dyn_quant_pair_flat_kernel<true, 1>), dim3((unsigned)fb), dim3(256), 0, s, x, M, K,
-                       (const float*)sample, kSpecSamples, q, e_out, erow, partial, guess);
-    hipLaunchKernelGGL((dyn_quant_pair_flat_kernel<true, 2>), dim3((unsigned)fb), dim3(256), 0, s, x, M, K,
-                       (const float*)partial, (int)fb, q, e_out, erow, (float*)nullptr, guess);
-    return lsk::check_launch("dyn_quant_pair_flat_kernel");
-  }
+  if (in_order && g_dynq == 1 && 4 * total >= kSpecBytes)
+    return launch_spec<true>(x, M, K, q, e_out, erow, partial, s);
   if (nt)
     hipLaunchKernelGGL(dyn_amax_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, s, x, M, K, ldx, flat, partial);
   else
@@ -758,10 +789,10 @@ int launch_quant8_dyn_pair(const float* x, int64_t M, int64_t K, int64_t ldx, in
   if (in_order) {
     if (nt)
       hipLaunchKernelGGL(dyn_quant_pair_flat_kernel<true>, dim3((unsigned)fb), dim3(256), 0, s, x, M, K,
-                         (const float*)partial, (int)blocks, q, e_out, erow, (float*)nullptr, (int32_t*)nullptr);
+                         (const float*)partial, (int)blocks, q, e_out, erow, (float*)nullptr, (SpecWords*)nullptr);
     else
       hipLaunchKernelGGL(dyn_quant_pair_flat_kernel<false>, dim3((unsigned)fb), dim3(256), 0, s, x, M, K,
-                         (const float*)partial, (int)blocks, q, e_out, erow, (float*)nullptr, (int32_t*)nullptr);
+                         (const float*)partial, (int)blocks, q, e_out, erow, (float*)nullptr, (SpecWords*)nullptr);
     return lsk::check_launch("dyn_quant_pair_flat_kernel");
   }
   int64_t qblocks = (M + 1) / 2;
@@ -780,7 +811,7 @@ LinDynWs lindyn_layout(int64_t M, int64_t K) {
   auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
   LinDynWs l;
   l.partial = 0;
-  l.erow = up((int64_t)(kDynBlocks + kSpecSamples + 1) * 4);  // the partial maxima, the sample's, the guess
+  l.erow = up((int64_t)kDynBlocks * 4 + (int64_t)sizeof(SpecWords));
   l.q = l.erow + up(M * 4);
   l.bytes = l.q + up(((M + 1) & ~(int64_t)1) * ((K + 63) / 64 * 64));
   return l;

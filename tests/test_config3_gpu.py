@@ -375,3 +375,55 @@ def test_linear_dyn_guessed_exponent(case, T, K, N):
     m = np.array([float(x.abs().max())], np.float32)
     assert int(e.item()) == int(e0.item()) == (0 if case == "all zero" else int(C._e_from_max(m)[0]))
     assert torch.equal(y.view(torch.int32), y0.view(torch.int32))
+
+
+@pytest.mark.parametrize("T,K,N", [(2050, 8256, 256), (1025, 16496, 256)])   # row pairs / rows
+@pytest.mark.parametrize("case", ["late", "first unsampled", "rising", "spread", "over", "zero sample", "inf"])
+def test_linear_dyn_guessed_exponent_put_right(case, T, K, N):
+    """The guess proven wrong along the way: by the last value, by the first the sample leaves out, by ever
+    larger ones all over (several lowerings a wave) or in one run; by headroom past a power of two that
+    the maximum stays under; over a sample of zeros; and by an infinity.  Exponent and result are the
+    two passes', the exponent the oracle's."""
+    from lockstep_amd import _lib as L
+    from lockstep_amd import ref_block_v1 as RB
+    say("guessed exponent put right", case)
+    g = torch.Generator(device=dev())
+    g.manual_seed(6)
+    x = torch.randn((T, K), generator=g, device=dev()).clamp_(-5.0, 5.0)
+    flat = x.view(-1)
+
+    def unsampled(at, step=1):               # the nearest element the sample's pieces leave out, past row 0
+        while True:
+            grp, piece = at >> 11, (at & 2047) >> 6
+            if at >= K and piece != ((grp * 0x9E3779B1) & 0xffffffff) >> 27:
+                return at
+            at += step
+    n = T * K
+    if case == "late":
+        flat[unsampled(n - 1, -1)] = 500.0
+    elif case == "first unsampled":
+        flat[unsampled(0)] = -500.0
+    elif case == "rising":
+        for j in range(40):
+            flat[unsampled(n * (j + 1) // 41)] = 8.5 * 2.0 ** (j // 4)
+    elif case == "spread":
+        for j in range(8):
+            flat[unsampled(n // 2 + 2100 * j)] = 8.5 * 2.0 ** j
+    elif case == "over":
+        x[:, ::32] = 4.5                     # (every piece holds one: the sample has headroom)
+        x[0, 5] = 7.9
+    elif case == "zero sample":
+        x.zero_()
+        flat[unsampled(n // 3)] = 3e-5
+    elif case == "inf":
+        flat[unsampled(n // 5)] = float("inf")
+    W = torch.randint(-127, 128, (N, K), generator=g, device=dev(), dtype=torch.int8)
+    y, e = RB.linear_dyn(x, W.t(), 7)
+    L.call("lsk_quant8_dyn_variant", 0)
+    try:
+        y0, e0 = RB.linear_dyn(x, W.t(), 7)
+    finally:
+        L.call("lsk_quant8_dyn_variant", 1)
+    m = np.array([float(x.abs().max())], np.float32)
+    assert int(e.item()) == int(e0.item()) == (-32 if case == "inf" else int(C._e_from_max(m)[0]))
+    assert torch.equal(y.view(torch.int32), y0.view(torch.int32))
