@@ -251,9 +251,10 @@ int lsk_gemm_select(int tile_id);
 /* No counterpart in the reference: bytes of room for K-split partial sums with which M rows, N output
  * channels and depth K are fastest (0 where no split is taken; no device work).  lsk_w8a8_matmul,
  * lsk_w8a8_outlier_linear and lsk_linear_dyn use whatever their workspace holds past the size their
- * own workspace query gives, so a caller adds this to it; with less room they split less or not at
- * all.  The same results. */
+ * own workspace query gives, so a caller adds this to it (lsk_outlier_split_bytes for the outlier
+ * linear, which rarely splits); with less room they split less or not at all.  The same results. */
 int64_t lsk_gemm_split_bytes(int64_t M, int64_t N, int64_t K);
+int64_t lsk_outlier_split_bytes(int64_t M, int64_t N, int64_t K);
 
 /* Tuning control with no counterpart in the reference: K slices of the tiles 0 and 20 when selected,
  * room permitting (0, the default: one).  Results are identical.  Thread-local. */

@@ -59,6 +59,7 @@ SIGNATURES = {
     "lsk_gemm_select": (_I, [_I]),
     "lsk_gemm_split": (_I, [_I]),
     "lsk_gemm_split_bytes": (_I64, [_I64, _I64, _I64]),
+    "lsk_outlier_split_bytes": (_I64, [_I64, _I64, _I64]),
     "lsk_gemm_skinny_shape": (_I, [_I, _I, _I]),
     "lsk_moe_skinny_shape": (_I, [_I, _I]),
     "lsk_moe_pp_skinny_rows": (_I, [_I]),

@@ -2246,11 +2246,15 @@ extern "C" int lsk_gemm_select(int tile_id) {
   return LSK_OK;
 }
 
-extern "C" int64_t lsk_gemm_split_bytes(int64_t M, int64_t N, int64_t K) {
+static int64_t split_room(int64_t M, int64_t N, int64_t K, bool v25) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 16 != 0) return 0;
   if (lsk::g_force_tile == 0 || lsk::g_force_tile == 20) return lsk::split_bytes(M, N, lsk::g_split);
-  return lsk::g_force_tile < 0 ? lsk::split_bytes(M, N, lsk::mid_plan(M, N, K, INT64_MAX).S) : 0;
+  return lsk::g_force_tile < 0 ? lsk::split_bytes(M, N, lsk::mid_plan(M, N, K, INT64_MAX, v25).S) : 0;
 }
+
+extern "C" int64_t lsk_gemm_split_bytes(int64_t M, int64_t N, int64_t K) { return split_room(M, N, K, false); }
+
+extern "C" int64_t lsk_outlier_split_bytes(int64_t M, int64_t N, int64_t K) { return split_room(M, N, K, true); }
 
 extern "C" int lsk_gemm_split(int n) {
   LSK_REQUIRE(n >= 0 && n <= 64, "lsk_gemm_split: %d slices not in [0, 64]", n);

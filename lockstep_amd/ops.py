@@ -166,7 +166,7 @@ def w8a8_outlier_linear(x2: torch.Tensor, oidx: torch.Tensor, wo: torch.Tensor, 
     if M == 0 or N == 0:
         return out
     lib = L.load()
-    nbytes = lib.lsk_w8a8_outlier_linear_workspace(M, K, ko) + lib.lsk_gemm_split_bytes(M, N, K)
+    nbytes = lib.lsk_w8a8_outlier_linear_workspace(M, K, ko) + lib.lsk_outlier_split_bytes(M, N, K)
     work = torch.empty((nbytes,), dtype=torch.uint8, device=x2.device)
     ws, bias = _f32(ws), _f32(bias)
     L.call("lsk_w8a8_outlier_linear", L.ptr(x2), xc, x2.stride(0) if M > 1 else max(K, 1), M, K, L.ptr(oi), ko,

@@ -115,3 +115,15 @@ def test_moe_forward_rejects_bad_kernel_choice():
         a = L.MoeArgs(T=1, H=16, I=16, E=1, k=1, select=sel, mx_select=mxsel)
         assert lib.lsk_moe_forward(ctypes.addressof(a), None) != 0
         assert b"select" in lib.lsk_last_error()
+
+
+def test_split_room_queries():
+    """Room for K-split partial sums: what each linear's own plan uses (the outlier linear's side term
+    makes it split less), 0 off the split's ranges; no device work."""
+    lib = L.load()
+    assert lib.lsk_gemm_split_bytes(43, 2048, 4096) > 0 == lib.lsk_outlier_split_bytes(43, 2048, 4096)
+    for query in (lib.lsk_gemm_split_bytes, lib.lsk_outlier_split_bytes):
+        room = query(72, 3584, 18944)
+        assert room > 0 and room % (72 * 3584 * 4) == 0
+        for M, N, K in ((0, 3584, 18944), (1, 3584, 18944), (4096, 3584, 18944), (72, 3584, 0), (72, 3584, 18950)):
+            assert query(M, N, K) == 0, (M, N, K)
