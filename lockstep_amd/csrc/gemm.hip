@@ -259,8 +259,10 @@ __device__ __forceinline__ void pp_epilogue_v25(const typename C::Acc& acc, cons
   }
 }
 
-// One dense tile (eight-wave ping-pong or four-wave main loop, MAIN); same operand contract and
-// tile order as gemm_i8_mfma_kernel.  The epilogue operands of the tile (asc / row exponents,
+// One dense tile (eight-wave ping-pong or four-wave main loop, MAIN): C[m, n] = sum_k A[m, k] * W[n, k]
+// with the epilogue applied per element.  A and W are K-contiguous with 16-byte aligned rows and
+// K % 16 == 0.  Logical tile ids walk M-fastest inside groups of LSK_GROUP_M M-tiles after the XCD
+// remap.  The epilogue operands of the tile (asc / row exponents,
 // ws, bias, column exponents) are loaded into registers before the main loop and parked in LDS
 // after it, so the epilogue itself touches global memory only to store.  V25 (the outlier epilogue)
 // is an instantiation of its own, so the other orders' kernels keep their registers and code size.

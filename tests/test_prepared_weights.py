@@ -10,7 +10,7 @@ from lockstep_amd import ops
 
 def test_gemm_row_pair_query():
     lib = L.load()
-    # one activation row streams W8 whole rows; mid row counts use the register-staged tile: no copy
+    # one activation row streams W8 whole rows; mid row counts read whole lines of W8 a K stage: no copy
     for M in (1, 4, 64, 128):
         assert lib.lsk_gemm_reads_row_pairs(M, 28672, 4096) == 0, M
     # decode rows of wide weights whose activations fit in LDS: the skinny GEMV streams the copy
