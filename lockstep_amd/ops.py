@@ -386,6 +386,7 @@ def row_pair_copies(weights, make=True):
     for an inference tensor (no version counter tells its updates), or with ROW_PAIR_COPIES off."""
     global row_pair_packs
     out, made = [], []
+    capturing = None
     for w_nk in weights:
         out.append(None)
         if not ROW_PAIR_COPIES or w_nk.dim() != 2 or w_nk.dtype != torch.int8:
@@ -394,8 +395,11 @@ def row_pair_copies(weights, make=True):
         if K == 0 or N == 0 or K % 16 != 0 or w_nk.stride(1) != 1 or w_nk.stride(0) % 16 != 0 \
                 or w_nk.data_ptr() % 16 != 0:
             continue
-        if w_nk.is_cuda and torch.cuda.is_current_stream_capturing():
-            continue
+        if w_nk.is_cuda:
+            if capturing is None:            # (256 copies of an expert list: asked once)
+                capturing = torch.cuda.is_current_stream_capturing()
+            if capturing:
+                continue
         owner, key = _pair_key(w_nk)
         if owner.is_inference():
             continue
